@@ -4,9 +4,8 @@
 //
 // Five launches:
 //   k_affine_rows   the affine projections qkv, z, b (beta) and a (decay) of the S rows in
-//                   one launch (q38_affine.hip): a workgroup takes a block of one projection's
-//                   weight rows for up to 16 staged rows; outputs rounded to bf16
-//                   (quantized_matmul's output);
+//                   one launch (q38_affine.hip), outputs rounded to bf16 (quantized_matmul's
+//                   output);
 //   k_gdn_prework   per (row, head): the depthwise width-4 convolution over [origin conv rows ;
 //                   qkv rows] and SiLU (T(c * T(sigmoid c))), the q / k RMS norms with the
 //                   1/DK and 1/sqrt(DK) scales, v, and per value head beta = T(sigmoid b) and
@@ -24,7 +23,8 @@
 //   k_affine_rows   the output projection.
 // A state (q38_gdn_state_bytes) is the conv rows [3][C] bf16 followed by the recurrent state
 // [HV][DV][DK] bf16, C = 2 HK DK + HV DV; value head h reads key head h / (HV / HK).
-#include "q38_affine.hpp"
+#include "q38_device.hpp"
+#include "q38_internal.hpp"
 
 namespace q38 {
 

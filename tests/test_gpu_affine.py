@@ -82,6 +82,17 @@ def test_affine_shared_layer_vs_oracle(layers, q38, orc, key, M):
     print(f"affine shared {key} M={M}: rel L2 {r:.2e}, max abs {m:.2e}")
 
 
+@pytest.mark.parametrize("key,M", [((8, 32, 1), 17), ((8, 32, 1), 70), ((2, 128, 0), 64), ((4, 64, 0), 65)])
+def test_affine_shared_row_tiles(layers, q38, orc, key, M):
+    """Row counts around the 64 request rows of a workgroup, whole and partial 512-input slabs."""
+    L = layers[key]
+    x = orc.rmsnorm(orc.embed(0x5EED + M, list(range(50, 50 + M)), 2048))
+    y, ex, wt, _, _ = run_forward(q38, L, L.qdesc, x)
+    wy, wex, wwt, _ = L.oracle(orc, x)
+    assert np.array_equal(ex, wex) and np.array_equal(wt, wwt)
+    tol_check(orc, y, wy)
+
+
 def test_affine_shared_prefill_width(layers, q38, orc):
     L = layers[(4, 64, 0)]
     M = 40

@@ -81,6 +81,29 @@ def test_verify_vs_oracle(gpu, q38, orc, geo, S):
         dev.close()
 
 
+@pytest.mark.parametrize("S", [1, 16, 17, 64])
+@pytest.mark.parametrize("geo", [
+    dict(hidden=672, hk=1, hv=3, dk=64, dv=64, bits=4, group=32),             # a 160-input slab, 3-row projections
+    dict(hidden=1152, hk=2, hv=6, dk=64, dv=64, bits=2, group=128, fmt=1),    # a slab of one group
+    dict(hidden=4160, hk=1, hv=1, dk=64, dv=64, bits=8, group=64),            # nine slabs over eight waves
+])
+def test_projection_tiles(gpu, q38, orc, geo, S):
+    """Projections whose inputs end inside a 512-input slab or need more slabs than waves, whose
+    outputs end inside a 16-row tile, at the row counts around the one- and four-tile kernels."""
+    L = GdnLayer(seed=21, **geo)
+    dev = DevGdn(q38, gpu, L)
+    try:
+        rng = np.random.default_rng(S)
+        x = orc.bf16(rng.normal(0, 1, (S, L.hidden)).astype(np.float32))
+        out, ck, _ = dev.verify(x)
+        wout, wck = orc.gdn_verify(L, x, None)
+        compare(orc, L, out, ck, wout, wck)
+        one, _, _ = dev.verify(x[:1])
+        assert np.array_equal(one[0], out[0])  # the same sums whatever the call's row count
+    finally:
+        dev.close()
+
+
 def test_full_size_layer(gpu, q38, orc):
     """The family's geometry: hidden 2048, 16 key and 32 value heads of 128, Q8/g64."""
     L = GdnLayer(hidden=2048, hk=16, hv=32, seed=4)
