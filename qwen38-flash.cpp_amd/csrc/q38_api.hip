@@ -1003,7 +1003,7 @@ static int check_forward_rows(const q38_moe_layer* L, int rows) {
     if (rows >= 1 && rows <= kMaxRows) return Q38_OK;
     if (rows < 1 || rows > kMaxPrefillRows) return fail(Q38_EINVAL, "rows must be between 1 and 2048");
     if (L->desc.top_k * rows > 32768) return fail(Q38_EINVAL, "rows x top_k must not exceed 32768");
-    if (!moe_supports_prefill(L->dev) && !moe_supports_grouped_prefill(L->dev))
+    if (!moe_supports_prefill(L->dev, rows) && !moe_supports_grouped_prefill(L->dev))
         return fail(Q38_EINVAL, "prefill widths (rows > 16) need a uniform layer of d8/14, d4/8 or d2/8 codes");
     return Q38_OK;
 }
@@ -1042,13 +1042,15 @@ int q38_moe_route(q38_moe_layer* L, const uint16_t* x, int32_t rows, const q38_r
 static int run_prefill(q38_moe_layer* L, const MoeBufs& w, int rows, const uint16_t* x, uint16_t* y,
                        const q38_route_out* trace, hipEvent_t* ev, hipStream_t st) {
     if (int rc = route_prefill(L, w, rows, x, st, ev)) return rc;
-    Q38_HIP(launch_shared_affine(L->dev, w, rows, st));
-    LayerDev one = expert_view(L->dev);  // partial-sum planes of the prefill kernels
+    const bool seg = moe_supports_prefill(L->dev, rows);
+    LayerDev all = L->dev;  // with the partial-sum planes of the prefill kernels
+    all.gu_parts = all.d_parts = seg ? prefill_planes(L->dev, rows) : 1;
+    Q38_HIP(launch_shared_affine(all, w, rows, st));
+    LayerDev one = expert_view(all);
     KernelTimer& kt = kernel_timer();
-    if (!moe_supports_prefill(L->dev)) {
-        // scale groups, d4 and d2 codes: the grouped kernels over 16-route passes of each slot
-        // (one partial-sum plane; SwiGLU inside the down kernel)
-        one.gu_parts = one.d_parts = 1;
+    if (!seg) {
+        // other scale groups, d4 and d2 codes: the grouped kernels over 16-route passes of each
+        // slot (one partial-sum plane; SwiGLU inside the down kernel)
         if (ev) kt = {ev[6], ev[7]};
         Q38_HIP(launch_gate_up_grouped(one, w, rows, st));
         kt = {};
@@ -1066,7 +1068,6 @@ static int run_prefill(q38_moe_layer* L, const MoeBufs& w, int rows, const uint1
         kt = {};
         return Q38_OK;
     }
-    one.gu_parts = one.d_parts = prefill_planes(L->dev, rows);
     if (ev) kt = {ev[6], ev[7]};
     Q38_HIP(launch_gate_up_pf(one, w, rows, st));
     if (trace)

@@ -322,7 +322,7 @@ int mfma_grid();  // persistent workgroups of the expert kernels (a multiple of 
 // Prefill widths, kMaxRows < M <= kMaxPrefillRows (q38_moe_pf.hip), one kernel each:
 // router logits, per-row top-k, sorted plan, segmented gate/up, SwiGLU, segmented down
 // (gate/up/down write one plane each).
-bool moe_supports_prefill(const LayerDev& L);
+bool moe_supports_prefill(const LayerDev& L, int M);
 hipError_t launch_router_rows(const LayerDev& L, const MoeBufs& B, int M, const uint16_t* x, hipStream_t st);
 hipError_t launch_topk_rows(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st);
 hipError_t launch_plan_sort(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st);

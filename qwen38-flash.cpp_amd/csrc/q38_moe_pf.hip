@@ -18,8 +18,8 @@
 //                  loaded while the current block is decoded and multiplied
 //   k_swiglu_pf    SwiGLU of every route with the reference's rounding points, fp16
 //   k_dn_pf        down segmented GEMM over the SwiGLU rows, same scheme
-// Row scales multiply the accumulated tile at the end. Layers: d8/14-bit, one scale per
-// output row, fp16 codebooks.
+// Row scales multiply the accumulated tile at the end; the LDS-codebook kernels also take one
+// scale per 64 inputs. Layers: d8/14-bit, fp16 codebooks.
 #include "q38_moe_dev.hpp"
 
 namespace q38 {
@@ -513,7 +513,7 @@ constexpr int kSegTab = 64;                      // units one workgroup walks (c
 struct SegTab {
     int32_t ustart[kSegMaxSlots + 1];
     int4 unit[kSegTab];                 // expert, route count, first sorted position, first route
-    int32_t row[kSegTab][kSegRoutes];   // per route of the unit (-1 past the slot's routes)
+    alignas(16) int32_t row[kSegTab][kSegRoutes];   // per route of the unit (-1 past the slot's routes)
 };
 
 __device__ __forceinline__ void seg_wait_vm() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
@@ -602,6 +602,21 @@ __device__ __forceinline__ void seg_load_codes(const uint32_t* codes_t, int KS, 
     }
 }
 
+// Chunks 0, 1 (half 0: words 0..7) or 2, 3 (half 1: words 8..13) of a row's block.
+__device__ __forceinline__ void seg_load_half(const uint32_t* codes_t, int KS, size_t tile64, int rr, int blk, int half,
+                                              uint32_t (&w)[14]) {
+    const uint32_t* base = codes_t + (tile64 * KS + blk) * (14 * 64);
+    const uint4 a = *reinterpret_cast<const uint4*>(base + 512 * half + rr * 4);
+    w[8 * half] = a.x; w[8 * half + 1] = a.y; w[8 * half + 2] = a.z; w[8 * half + 3] = a.w;
+    if (half == 0) {
+        const uint4 b = *reinterpret_cast<const uint4*>(base + 256 + rr * 4);
+        w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
+    } else {
+        const uint2 b = *reinterpret_cast<const uint2*>(base + 768 + rr * 2);
+        w[12] = b.x; w[13] = b.y;
+    }
+}
+
 // 8 x code q of a packed 32-code block (the LDS byte offset of its 4-dim entry): one shift
 // (or funnel shift, for a code that spans two words) and one mask.
 __device__ __forceinline__ uint32_t code14_x8(const uint32_t* w, int q) {
@@ -641,6 +656,122 @@ __device__ __forceinline__ void seg_mfma(const uint32_t (&w)[2][NW], const uint4
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// ---- scale groups of 64 inputs (8 subvectors; the reference checkpoints' layout)
+// A group's sum must meet one scale, so one MFMA takes the 32 chunk dims of one group: lane
+// quarter q its subvectors 2 q, 2 q + 1. The lanes load code blocks as above (quarter q the
+// q-th span of SPL codes of the K part), cut them into pairs of codes (28 bits) and transpose
+// the pairs over the quarters with lane swaps: pair p of group g of span b goes to quarter p,
+// the group's register. The operands trade places against
+// the per-row kernels: A = the route rows, B = the weights, so that a lane owns one weight row
+// (column lane & 15), reads that row's scales, and holds its products with routes 4 q .. 4 q + 3.
+// Bound like the per-row kernels by the random LDS gathers, then by the four scaled adds per
+// MFMA. At 2048 rows (512 experts of about 40 routes): gate/up 6,883 -> 330 us and down 2,862
+// -> 205 us against the grouped vector kernels, which still take the other group sizes.
+// (Two groups of each span at a time: w holds their 7 words, pr the four spans' pairs, pair
+// 2 b + g for group g of span b.)
+__device__ __forceinline__ void seg_pairs(const uint32_t (&w)[7], uint32_t (&pr)[8]) {
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        uint32_t r[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int bit = 28 * (4 * g + p), wi = bit >> 5, sh = bit & 31;
+            r[p] = sh + 28 > 32 ? __builtin_amdgcn_alignbit(w[wi + 1], w[wi], sh) : w[wi] >> sh;
+        }
+        const auto a = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
+        const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+        const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+        pr[g] = c[0];
+        pr[2 + g] = c[1];
+        pr[4 + g] = d[0];
+        pr[6 + g] = d[1];
+    }
+}
+
+// Two 16-row tiles of one item over 8 groups, group gid(j) for pair j: acc[i] += scale * (A =
+// routes bx[gid]) x (B = the gathered pair of tile i). sc: the lane's row scales of the K part,
+// two groups per word. The gathers run LA MFMAs ahead, the scaled adds two MFMAs behind.
+template <int NG, typename F>
+__device__ __forceinline__ void seg_mfma_g8(const uint32_t (&pr)[2][8], const uint4 (&bx)[NG],
+                                            const uint32_t (&sc)[2][NG / 2], const unsigned char* book, F gid,
+                                            f4_t (&acc)[2]) {
+    constexpr int NM = 16, LA = 4, LAG = 2;
+    uint4 a[NM];
+    f4_t d[NM];
+    auto gather = [&](int m) {
+        const uint32_t v = pr[m & 1][m >> 1];
+        const uint2 a0 = *reinterpret_cast<const uint2*>(book + ((v << 3) & 0x1FFF8u));
+        const uint2 a1 = *reinterpret_cast<const uint2*>(book + ((v >> 11) & 0x1FFF8u));
+        a[m] = make_uint4(a0.x, a0.y, a1.x, a1.y);
+    };
+    auto add = [&](int m) {
+        const int g = gid(m >> 1);
+        const float s = h2f(static_cast<uint16_t>(g & 1 ? sc[m & 1][g >> 1] >> 16 : sc[m & 1][g >> 1]));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[m & 1][i] = fmaf(s, d[m][i], acc[m & 1][i]);
+    };
+#pragma unroll
+    for (int m = 0; m < LA; ++m) gather(m);
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (m + LA < NM) gather(m + LA);
+        d[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, bx[gid(m >> 1)]),
+                                                      __builtin_bit_cast(h8_t, a[m]), f4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if (m >= LAG) add(m - LAG);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = NM - LAG; m < NM; ++m) add(m);
+    // (without this the adds would be sunk to the sums' uses, past the end of the loop, and every
+    // MFMA result kept in registers until then)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(acc[i]));
+}
+
+// The products of one item (NSUB-independent): codes w of its two 16-row tiles (SPL 32: the
+// lane's 14 words, SPL 16: its 7), the next item's words loaded into w by next(half) as soon as
+// a half has become pairs.
+template <int SPL, int NG, typename F>
+__device__ __forceinline__ void seg_item_g8(uint32_t (&w)[2][SPL == 32 ? 14 : 7], const uint4 (&bx)[NG],
+                                            const uint32_t (&sc)[2][NG / 2], const unsigned char* book, F next,
+                                            f4_t (&acc)[2]) {
+    uint32_t pr[2][8];
+    if constexpr (SPL == 16) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) seg_pairs(w[i], pr[i]);
+        __builtin_amdgcn_sched_barrier(0);
+        next(0);
+        seg_mfma_g8<NG>(pr, bx, sc, book, [](int j) { return j; }, acc);
+    } else {
+        uint32_t w7[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t h[7] = {w[i][0], w[i][1], w[i][2], w[i][3], w[i][4], w[i][5], w[i][6]};
+            seg_pairs(h, pr[i]);
+            w7[i] = w[i][7];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        next(0);
+        seg_mfma_g8<NG>(pr, bx, sc, book, [](int j) { return 4 * (j >> 1) + (j & 1); }, acc);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t h[7] = {w7[i], w[i][8], w[i][9], w[i][10], w[i][11], w[i][12], w[i][13]};
+            seg_pairs(h, pr[i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        next(1);
+        seg_mfma_g8<NG>(pr, bx, sc, book, [](int j) { return 4 * (j >> 1) + 2 + (j & 1); }, acc);
+    }
+}
+
+// N fp16 scales at p (2-byte aligned) as packed pairs.
+template <int N>
+__device__ __forceinline__ void seg_load_scales(const uint16_t* p, uint32_t (&sc)[N / 2]) {
+    __builtin_memcpy(sc, p, N * 2);
+}
+
 __device__ __forceinline__ float4 seg_scaled(uint2 sc, const f4_t& a) {
     return make_float4(h2f(static_cast<uint16_t>(sc.x)) * a[0], h2f(static_cast<uint16_t>(sc.x >> 16)) * a[1],
                        h2f(static_cast<uint16_t>(sc.y)) * a[2], h2f(static_cast<uint16_t>(sc.y >> 16)) * a[3]);
@@ -656,7 +787,8 @@ __device__ __forceinline__ void seg_range(int n_items, int per_type, int idx, in
 // four K parts would not fit in LDS beside the 128 KiB codebook chunk). Output rows of an item:
 // TR = 32 * RG rows of I; chunk `chunk` of projection `proj` per workgroup type. B = rows of
 // the chunk-planar fp16 inputs ([2][M][H / 2]).
-template <int NSUB>
+// G8: one scale per 64 inputs (ngrp = H / 64) instead of one per output row.
+template <int NSUB, bool G8>
 __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, int M) {
     constexpr int KP = NSUB / 128, RG = 8 / KP, TR = 32 * RG, KS = NSUB / 32;
     static_assert(NSUB % 128 == 0 && KP * RG == 8, "8 waves = K parts x row groups");
@@ -703,14 +835,15 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
     float* out = (proj == 0 ? B.g : B.u) + chunk * B.gu_plane;
     const uint16_t* xplane = B.x16 + static_cast<size_t>(chunk) * M * (H / 2);
 
-    // B operand of unit k: request row T.row[k][r16], subvectors kh * 128 + 32 q + (0..31)
+    // x operand of unit k: request row T.row[k][r16], subvectors kh * 128 + 32 q + (0..31), 16
+    // bytes of two each; G8: subvectors 2 q, 2 q + 1 of each of the K part's 16 groups
     auto load_b = [&](int k, uint4 (&bx)[16]) {
         const int row = T.row[k][r16];
         if (row >= 0) {
             const uint4* src = reinterpret_cast<const uint4*>(xplane + static_cast<size_t>(row) * (H / 2) +
-                                                              (kh * 128 + 32 * q) * 4);
+                                                              (kh * 128 + (G8 ? 2 : 32) * q) * 4);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) bx[i] = src[i];
+            for (int i = 0; i < 16; ++i) bx[i] = src[G8 ? 4 * i : i];
         } else {
 #pragma unroll
             for (int i = 0; i < 16; ++i) bx[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -723,6 +856,70 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
             seg_load_codes<32>(P.codes_t, KS, row0 >> 6, static_cast<int>(row0 & 63) + 16 * i + r16, kh * 4 + q, 0,
                                w[i]);
     };
+    if constexpr (G8) {
+        auto load_scales = [&](int expert, int tile, uint32_t (&sc)[2][8]) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                seg_load_scales<16>(P.scales + (static_cast<size_t>(expert) * I + tile * TR + rg * 32 + 16 * i + r16) *
+                                                   (NSUB / 8) + kh * 16, sc[i]);
+        };
+        uint4 bx[16];
+        uint32_t w[2][14], sn[2][8];
+        int k = 0, tile = i0 - u0 * tiles;
+        load_b(0, bx);
+        load_codes(T.unit[0].x, tile, w);
+        load_scales(T.unit[0].x, tile, sn);
+        // an item's code words become pairs and its scales move over, then the next item's words
+        // and scales are requested into the same registers, then the products run
+        for (int item = i0; item < i1; ++item) {
+            const int4 un = T.unit[k];
+            const int o0 = tile * TR + rg * 32 + r16;
+            const bool last = item + 1 >= i1;
+            const bool new_unit = !last && tile + 1 == tiles;
+            const int ne = new_unit ? T.unit[k + 1].x : un.x, nt = last ? tile : new_unit ? 0 : tile + 1;
+            uint32_t sc[2][8];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int v = 0; v < 8; ++v) sc[i][v] = sn[i][v];
+            f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
+            seg_item_g8<32, 16>(w, bx, sc, book, [&](int half) {
+                const size_t row0 = static_cast<size_t>(ne) * I + nt * TR + rg * 32;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    seg_load_half(P.codes_t, KS, row0 >> 6, static_cast<int>(row0 & 63) + 16 * i + r16, kh * 4 + q, half,
+                                  w[i]);
+                if (half == 0) load_scales(ne, nt, sn);
+            }, acc);
+            if (new_unit) load_b(k + 1, bx);
+            const int buf = item & 1;
+            if (KP > 1) {
+                if (kh > 0)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) red[(((buf * (KP - 1) + kh - 1) * RG + rg) * 2 + i) * 64 + lane] = acc[i];
+                lds_barrier();
+            }
+            if (kh == 0)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    f4_t sum = acc[i];
+#pragma unroll
+                    for (int p = 1; p < KP; ++p) sum += red[(((buf * (KP - 1) + p - 1) * RG + rg) * 2 + i) * 64 + lane];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int j = un.w + 4 * q + v;
+                        if (j < un.y) out[static_cast<size_t>(un.z + j) * I + o0 + 16 * i] = sum[v];
+                    }
+                }
+            if (new_unit) {
+                ++k;
+                tile = 0;
+            } else {
+                ++tile;
+            }
+        }
+        return;
+    }
     uint4 bx[16];
     load_b(0, bx);
     // (k, tile): the current item's unit (table index) and tile, advanced without divisions
@@ -782,7 +979,7 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
 // half a code block). One K part: wave rg owns rows 32 rg .. + 31 of a TR = 256-row tile of
 // H. B = the pass's SwiGLU rows (chunk-planar fp16 at sorted positions); outputs at the
 // route index.
-template <int NSUB>
+template <int NSUB, bool G8>
 __global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, int M) {
     constexpr int SPL = NSUB / 4, TR = 256, KS = NSUB / 32;
     static_assert(SPL == 16 || SPL == 32, "16-code or 32-code lane spans");
@@ -827,16 +1024,16 @@ __global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, i
     const uint16_t* hplane = B.h16 + static_cast<size_t>(chunk) * MKM * (I / 2);
     const int blk = SPL * q / 32, half = SPL == 16 ? (q & 1) : 0;
 
-    // B operand of unit k: SwiGLU row (sorted position) of route j0 + r16, subvectors
-    // SPL q + (0..SPL-1)
+    // SwiGLU operand of unit k: row (sorted position) of route j0 + r16, subvectors SPL q +
+    // (0..SPL-1), 16 bytes of two each; G8: subvectors 2 q, 2 q + 1 of each group
     auto load_b = [&](int k, uint4 (&bx)[NB]) {
         const int4 un = T.unit[k];
         const int j = un.w + r16;
         if (j < un.y) {
-            const uint4* src =
-                reinterpret_cast<const uint4*>(hplane + static_cast<size_t>(un.z + j) * (I / 2) + SPL * q * 4);
+            const uint4* src = reinterpret_cast<const uint4*>(hplane + static_cast<size_t>(un.z + j) * (I / 2) +
+                                                              (G8 ? 2 : SPL) * q * 4);
 #pragma unroll
-            for (int i = 0; i < NB; ++i) bx[i] = src[i];
+            for (int i = 0; i < NB; ++i) bx[i] = src[G8 ? 4 * i : i];
         } else {
 #pragma unroll
             for (int i = 0; i < NB; ++i) bx[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -849,6 +1046,60 @@ __global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, i
             seg_load_codes<SPL>(P.codes_t, KS, row0 >> 6, static_cast<int>(row0 & 63) + 16 * i + r16, blk, half,
                                 w[i]);
     };
+    if constexpr (G8) {
+        auto load_scales = [&](int expert, int tile, uint32_t (&sc)[2][NB / 2]) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                seg_load_scales<NB>(P.scales + (static_cast<size_t>(expert) * H + tile * TR + rg * 32 + 16 * i + r16) * NB,
+                                    sc[i]);
+        };
+        uint4 bx[NB];
+        uint32_t w[2][NW], sn[2][NB / 2];
+        int k = 0, tile = i0 - u0 * tiles;
+        load_b(0, bx);
+        load_codes(T.unit[0].x, tile, w);
+        load_scales(T.unit[0].x, tile, sn);
+        for (int item = i0; item < i1; ++item) {
+            const int expert = T.unit[k].x;
+            const int4 rt = *reinterpret_cast<const int4*>(&T.row[k][4 * q]);  // routes 4 q .. 4 q + 3 (-1: none)
+            const int o0 = tile * TR + rg * 32 + r16;
+            const bool last = item + 1 >= i1;
+            const bool new_unit = !last && tile + 1 == tiles;
+            const int ne = new_unit ? T.unit[k + 1].x : expert, nt = last ? tile : new_unit ? 0 : tile + 1;
+            uint32_t sc[2][NB / 2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int v = 0; v < NB / 2; ++v) sc[i][v] = sn[i][v];
+            f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
+            seg_item_g8<SPL, NB>(w, bx, sc, book, [&](int half) {
+                if constexpr (SPL == 16) {
+                    load_codes(ne, nt, w);
+                } else {
+                    const size_t row0 = static_cast<size_t>(ne) * H + nt * TR + rg * 32;
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        seg_load_half(P.codes_t, KS, row0 >> 6, static_cast<int>(row0 & 63) + 16 * i + r16, blk, half,
+                                      w[i]);
+                }
+                if (half == 0) load_scales(ne, nt, sn);
+            }, acc);
+            if (new_unit) load_b(k + 1, bx);
+            const int rts[4] = {rt.x, rt.y, rt.z, rt.w};
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (rts[v] >= 0) dout[static_cast<size_t>(rts[v]) * H + o0 + 16 * i] = acc[i][v];
+            if (new_unit) {
+                ++k;
+                tile = 0;
+            } else {
+                ++tile;
+            }
+        }
+        return;
+    }
     uint4 bx[NB];
     load_b(0, bx);
     int k = 0, tile = i0 - u0 * tiles;
@@ -931,10 +1182,15 @@ hipError_t launch_router_rows_t(const LayerDev& L, const MoeBufs& B, int M, cons
 
 } // namespace
 
-bool moe_supports_prefill(const LayerDev& L) {
+bool moe_supports_prefill(const LayerDev& L, int M) {
     if (L.mixed) return false;
-    for (int p = 0; p < 3; ++p)
-        if (L.p[p].dim != 8 || L.p[p].bits != 14 || L.p[p].ngrp != 1 || !L.p[p].book) return false;
+    bool groups = false;
+    for (int p = 0; p < 3; ++p) {
+        if (L.p[p].dim != 8 || L.p[p].bits != 14 || !L.p[p].book) return false;
+        groups |= L.p[p].ngrp != 1;
+    }
+    // (scale groups: on the LDS-codebook kernels only; the tile kernels scale whole rows)
+    if (groups && prefill_planes(L, M) != 2) return false;
     return L.H % kPfK == 0 && L.I % kPfK == 0 && L.H % kPfRows == 0 && L.I % kPfRows == 0 && L.H % 512 == 0 &&
            L.H <= 4096 && L.E <= 65535;
 }
@@ -975,15 +1231,20 @@ static int pf_slots(const LayerDev& L, int M) {
 // its table; others take the tile kernels.
 static int64_t seg_units_per_wg(const LayerDev& L, int M, int tiles, int per_type) {
     const int64_t MK = static_cast<int64_t>(M) * L.K;
-    const int64_t ns = (MK < L.E ? MK : L.E) + (L.has_shared ? 1 : 0);
-    const int64_t units = (MK + (L.has_shared ? M : 0) + (kSegRoutes - 1) * ns) / kSegRoutes;  // >= sum ceil(n/16)
+    const int shared = L.has_shared && !L.shared_affine;  // (an affine shared expert has no slot)
+    const int64_t ns = (MK < L.E ? MK : L.E) + shared;
+    const int64_t units = (MK + (shared ? M : 0) + (kSegRoutes - 1) * ns) / kSegRoutes;  // >= sum ceil(n/16)
     const int64_t items = (units * tiles + per_type - 1) / per_type;
     return (items + tiles - 1) / tiles + 1;
 }
 
 int prefill_planes(const LayerDev& L, int M) {
-    for (int p = 0; p < 3; ++p)
+    for (int p = 0; p < 3; ++p) {
         if (!L.p[p].book4 || !L.p[p].codes_t) return 1;
+        // one scale per row or per 64 inputs
+        if (L.p[p].ngrp != 1 && L.p[p].ngrp * 64 != (p < 2 ? L.H : L.I)) return 1;
+    }
+    if (L.p[0].ngrp != L.p[1].ngrp) return 1;
     const int gn = L.H / 8, dn = L.I / 8;
     if ((gn != 128 && gn != 256) || (dn != 64 && dn != 128)) return 1;
     const int gu_rows = 32 * (8 / (gn / 128));  // output rows of a gate/up item
@@ -997,11 +1258,13 @@ int prefill_planes(const LayerDev& L, int M) {
 
 template <int NSUB>
 hipError_t launch_gu_seg_t(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
-    return launch(k_gu_seg<NSUB>, dim3(mfma_grid()), dim3(kSegThreads), 0, st, L, B, M);
+    return launch(L.p[0].ngrp > 1 ? k_gu_seg<NSUB, true> : k_gu_seg<NSUB, false>, dim3(mfma_grid()), dim3(kSegThreads), 0,
+                  st, L, B, M);
 }
 template <int NSUB>
 hipError_t launch_dn_seg_t(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
-    return launch(k_dn_seg<NSUB>, dim3(mfma_grid()), dim3(kSegThreads), 0, st, L, B, M);
+    return launch(L.p[2].ngrp > 1 ? k_dn_seg<NSUB, true> : k_dn_seg<NSUB, false>, dim3(mfma_grid()), dim3(kSegThreads), 0,
+                  st, L, B, M);
 }
 
 hipError_t launch_gate_up_pf(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {

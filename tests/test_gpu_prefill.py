@@ -195,6 +195,25 @@ def test_prefill_512_zipf_group64(gpu, q38, orc):
         L.close()
 
 
+@pytest.mark.parametrize("groups", [(64, 64), (64, None), (None, 64)])
+@pytest.mark.parametrize("M", [17, 33])
+def test_prefill_group64_segments(gpu, q38, orc, groups, M):
+    """Scale groups in both projections or in one of them on the LDS-codebook kernels, at row
+    counts where most units hold one route and the shared slot ends in a unit of one: every row
+    against the oracle."""
+    geo = dict(gu_group=groups[0], down_group=groups[1])
+    L = q38.MoeLayer(gpu, q38.desc(**geo), seed=SEED, layer=LAYER)
+    try:
+        x = orc.rmsnorm(orc.embed(SEED, tokens(M), 2048))
+        y, ex, wt, lg, plan = run_forward(q38, L, q38.desc(**geo), x)
+        wy, wex, wwt, _ = orc.moe_layer_synth(oracle_lib.make_desc(**geo), SEED, LAYER, x)
+        assert np.array_equal(ex, wex) and np.array_equal(wt.view(np.uint32), wwt.view(np.uint32))
+        stable_plan_check(orc, plan, ex, 512)
+        tol_check(orc, y, wy)
+    finally:
+        L.close()
+
+
 @pytest.mark.parametrize("geo,M", [(dict(gu=(4, 8), down=(4, 8)), 40), (dict(gu=(2, 8), down=(2, 8), gu_group=64,
                                                                             down_group=64), 100),
                                    (dict(gu=(8, 14), down=(4, 8), gu_group=64, down_group=64), 33)])
