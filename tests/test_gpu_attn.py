@@ -153,6 +153,34 @@ def test_rows_chain_through_the_cache(gpu, q38):
         dev.close()
 
 
+@pytest.mark.parametrize("geo,S,T0", [
+    (dict(), 5, 16381),                                          # rows on both sides of the first P.V tile limit
+    (dict(head_dim=64, rotary_dim=64), 5, 24573),                # and of the second
+    (dict(q_heads=16, head_dim=64, rotary_dim=32), 64, 8200),    # several score tiles per workgroup
+    (dict(q_heads=8, kv_heads=1, head_dim=256, rotary_dim=64), 5, 130),   # 40 queries: a partial chunk
+])
+def test_tile_variants(gpu, q38, orc, geo, S, T0):
+    """The score and P.V kernels' tile sizes, against the oracle and, bit for bit, against one-row
+    calls of the first and last row."""
+    L = AttnLayer(seed=9, **geo)
+    rng = np.random.default_rng(T0)
+    cap = T0 + S + 3
+    keys, values = L.random_cache(rng, cap, T0)
+    x = to16(rng.normal(0, 1, (S, L.hidden)), 0)
+    dev = DevAttn(q38, gpu, L, cap)
+    try:
+        cache = dev.cache_dev(keys, values)
+        out = dev.verify(x, cache, T0, T0)
+        k2, v2 = dev.cache_host(cache)
+        for r in (0, S - 1):
+            assert np.array_equal(dev.verify(x[r:r + 1], cache, T0 + r, T0 + r)[0], out[r]), r
+    finally:
+        dev.close()
+    wout, wk, wv = orc.attn_verify(L, x, keys, values, T0, T0)
+    tol_check(orc, out, wout)
+    check_cache(keys, values, k2, v2, wk, wv, T0, S)
+
+
 def test_one_hot_query_reads_its_key_exactly(gpu, q38, orc):
     j = 40
     L = identity_layer(q_rows={j: (0, 3)})
