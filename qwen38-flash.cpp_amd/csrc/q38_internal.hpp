@@ -137,10 +137,13 @@ struct LayerDev {
     AffineDev sa[3];
     int shared_affine, sa_bits, sa_group, sa_inter, sa_f16;
     // u8_native: the three projections carry U8 books the U8 verify kernels read (d8/14-bit,
-    // H 2048, I 512, per-row scales, no affine shared expert). u8_call: this call runs them
-    // (moe_call_dev: 1-16 rows while they are enabled); it then writes one partial-sum plane.
-    int u8_native, u8_call;
+    // H 2048, I 512, per-row scales, no affine shared expert). call_path: the kernels of this
+    // verify call (moe_call_dev). kPathU8: those (1-16 rows while they are enabled), one
+    // partial-sum plane; kPathSeg: the segmented LDS-codebook kernels of the prefill widths (5-16
+    // rows), two planes, the router storing the fp16 rows chunk-planar; kPathOther: the others.
+    int u8_native, call_path;
 };
+enum { kPathOther = 0, kPathU8 = 1, kPathSeg = 2 };
 
 // The view of a layer the routed-expert kernels take: without the shared slot when the shared
 // expert is affine (its down rows come from launch_shared_affine).
@@ -284,6 +287,8 @@ bool moe_plans_in_gate_up(const LayerDev& L, int M);
 // and d8 layers of the same geometry with per-64-input scale groups. They write one partial-
 // sum plane per codebook chunk (gu_parts / d_parts of the call: moe_call_dev).
 bool moe_uses_narrow(const LayerDev& L, int M);
+// Verify widths of 5-16 rows on the segmented kernels (q38_moe_pf.hip).
+bool moe_uses_seg_verify(const LayerDev& L, int M);
 // The layer view of a call of M rows: the partial-sum plane counts of the kernels it takes.
 LayerDev moe_call_dev(const LayerDev& L, int M);
 // Verify widths (1-16 rows) of layers with U8 books on the kernels that read the books

@@ -210,12 +210,14 @@ __global__ __launch_bounds__(1024) void k_prepare_u8(const uint16_t* __restrict_
 // (t outer, j inner) with fmaf, then the xor butterfly and BF16 rounding; a router bias,
 // when set, is added to the rounded logit in float. Workgroup 0 stores x in the workspace
 // (bf16) with its fp16 copy (the MFMA operand) unless src already is that copy.
-// reset_gu: the gate/up and down chunk planes of the call ([2][M*K + M][I] each for g and u,
+// flags, bit 0: the gate/up and down chunk planes of the call ([2][M*K + M][I] each for g and u,
 // [2][M*K + M][H] for d) are set to the all-ones pattern that the fused layer kernel (k_gd4)
-// waits on.
+// waits on. Bit 1: the fp16 copy is chunk-planar ([2][M][H / 2]: dims 4c..4c+3 of every
+// subvector in plane c), as the segmented kernels read it.
 template <int T, bool NORM, int MR>
 __global__ __launch_bounds__(128 * T) void k_route_norm(LayerDev L, MoeBufs B, int M, const uint16_t* __restrict__ src,
-                                                        float eps, int reset_gu) {
+                                                        float eps, int flags) {
+    const bool reset_gu = flags & 1, planar = MR > 4 && (flags & 2);  // (5-16 rows only)
     constexpr int H = 512 * T, NT = 128 * T, NW = NT / 64;
     extern __shared__ __align__(16) uint16_t xs[];  // [M][H] bf16
     __shared__ float red[MR][NW];
@@ -273,7 +275,9 @@ __global__ __launch_bounds__(128 * T) void k_route_norm(LayerDev L, MoeBufs B, i
                     xs[at] = b;
                     if (store) {
                         B.x[at] = b;
-                        B.x16[at] = f2h(bf2f(b));
+                        const int c = tid + NT * i;
+                        B.x16[planar ? (static_cast<size_t>((c >> 2) & 1) * M + r) * (H / 2) + (c >> 3) * 4 + (c & 3) : at] =
+                            f2h(bf2f(b));
                     }
                 }
             }
@@ -290,7 +294,12 @@ __global__ __launch_bounds__(128 * T) void k_route_norm(LayerDev L, MoeBufs B, i
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
                     hq[k] = static_cast<uint32_t>(f2h(bflo(q[k]))) | (static_cast<uint32_t>(f2h(bfhi(q[k]))) << 16);
-                reinterpret_cast<uint4*>(B.x16)[i] = make_uint4(hq[0], hq[1], hq[2], hq[3]);
+                if (planar) {  // (8 columns from 8 (i % (H / 8)) of row i / (H / 8): one subvector)
+                    reinterpret_cast<uint2*>(B.x16)[i] = make_uint2(hq[0], hq[1]);
+                    reinterpret_cast<uint2*>(B.x16)[static_cast<size_t>(M) * (H / 8) + i] = make_uint2(hq[2], hq[3]);
+                } else {
+                    reinterpret_cast<uint4*>(B.x16)[i] = make_uint4(hq[0], hq[1], hq[2], hq[3]);
+                }
             }
         }
     }
@@ -329,9 +338,82 @@ __global__ __launch_bounds__(128 * T) void k_route_norm(LayerDev L, MoeBufs B, i
     Q38_STAMP(0, 3);
 }
 
+// Plan (R3) of up to 16 rows x K <= 16 routes over 512 experts from t.ex, plan_wave's method over
+// a workgroup of at least 256 threads: thread (row, w) forms the mask and the prefix count of its
+// row's experts in [32 w, 32 w + 32); a route then adds up the rows' counts below its expert (16
+// LDS reads, where comparing it with every other route takes MK).
+__device__ __forceinline__ void plan_block512(int M, int K, const int32_t* ex, int32_t* plan) {
+    __shared__ uint32_t mask[kMaxRows][16], pref[kMaxRows][16];
+    const int tid = threadIdx.x, lane = tid & 63, MK = M * K;
+    if (tid < 256) {
+        const int mr = tid >> 4, mw = tid & 15;
+        uint32_t m = 0;
+        for (int s = 0; s < K; ++s) {
+            const int e = ex[(mr < M ? mr : 0) * K + s];
+            m |= (e >> 5) == mw ? 1u << (e & 31) : 0u;
+        }
+        if (mr >= M) m = 0;
+        const uint32_t pc = static_cast<uint32_t>(__popc(m));
+        mask[mr][mw] = m;
+        pref[mr][mw] = row_scan_incl(pc) - pc;
+    }
+    lds_barrier();
+    if (tid >= (MK + 63) / 64 * 64) return;  // (whole waves)
+    uint32_t u = 0;
+#pragma unroll
+    for (int r = 0; r < kMaxRows; ++r) u |= mask[r][lane & 15];
+    const uint32_t uc = static_cast<uint32_t>(__popc(u));
+    const uint32_t upref = row_scan_incl(uc) - uc;
+    const int nu = static_cast<int>(__builtin_amdgcn_readlane(static_cast<int>(upref + uc), 15));
+    const bool act = tid < MK;
+    const int e = act ? ex[tid] : 0, r = tid / K, w = e >> 5, b = e & 31;
+    const uint32_t low = (1u << b) - 1u;
+    int pos = 0, rank = 0;
+#pragma unroll
+    for (int rr = 0; rr < kMaxRows; ++rr) {
+        const uint32_t mk = mask[rr][w];
+        pos += static_cast<int>(pref[rr][w]) + __popc(mk & low);
+        rank += (rr < r && ((mk >> b) & 1u)) ? 1 : 0;
+    }
+    pos += rank;
+    const int urank = static_cast<int>(__shfl(static_cast<int>(upref), w, 64)) +
+                      __popc(static_cast<uint32_t>(__shfl(static_cast<int>(u), w, 64)) & low);
+    if (act) {
+        plan[2 + 2 * MK + pos] = tid;  // route at sorted position pos
+        plan[2 + 3 * MK + tid] = pos;  // sorted position of route tid
+        if (rank == 0) {
+            plan[1 + urank] = e;
+            plan[1 + MK + urank] = pos;
+        }
+        if (tid >= nu) {  // entries past the unique experts (every entry is written)
+            plan[1 + tid] = -1;
+            plan[1 + MK + tid + 1] = MK;
+        }
+    }
+    if (tid == 0) {
+        plan[0] = nu;
+        plan[1 + MK + nu] = MK;
+    }
+}
+
+// Top-k and plan of up to 16 rows in one workgroup; F512: 512 experts, one wave per row on the
+// counting top-k (13.5 -> 7.1 us at 13 rows, against the tournament and the pairwise plan).
+template <bool F512>
 __global__ __launch_bounds__(1024) void k_topk_plan(LayerDev L, MoeBufs B, int M) {
     __shared__ TopkLds t;
-    topk_plan_block(L, B, M, true, B.plan, t, 0);
+    if constexpr (F512) {
+        __shared__ __align__(16) uint64_t cand[16][64];
+        const int wave = threadIdx.x >> 6;
+        if (wave < M) {
+            float lg[8];
+            topk_load_row_t<8, true>(L, B, wave, lg);
+            topk_select_row_fast<8>(L, B, wave, lg, t.ex, true, cand[wave]);
+        }
+        lds_barrier();
+        plan_block512(M, L.K, t.ex, B.plan);
+    } else {
+        topk_plan_block(L, B, M, true, B.plan, t, 0);
+    }
 }
 
 // ============================================================== MFMA expert projections
@@ -1170,7 +1252,7 @@ hipError_t launch_route_norm_t(const LayerDev& L, const MoeBufs& B, int M, const
     const int rows = L.E + (L.has_shared ? 1 : 0);
     const int reset = moe_uses_fused(L, M) ? 1 : 0;
     return launch(k_route_norm<T, NORM, MR>, dim3((rows + NW - 1) / NW), dim3(128 * T), lds, st, L, B, M, src, eps,
-                  reset);
+                  reset | (L.call_path == kPathSeg ? 2 : 0));
 }
 template <int T, bool NORM>
 hipError_t launch_route_norm_m(const LayerDev& L, const MoeBufs& B, int M, const uint16_t* src, float eps,
@@ -1254,6 +1336,7 @@ bool moe_mixed_mfma(const LayerDev& L) {
 }
 
 bool moe_plans_in_gate_up(const LayerDev& L, int M) {
+    if (L.call_path == kPathSeg) return false;
     return moe_uses_mfma(L) || moe_mixed_mfma(L) || moe_uses_narrow(L, M);
 }
 
@@ -1291,7 +1374,11 @@ hipError_t launch_router(const LayerDev& L, const MoeBufs& B, int M, const uint1
 }
 
 hipError_t launch_topk_plan(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
-    return launch(k_topk_plan, dim3(1), dim3(1024), 0, st, L, B, M);
+    if (L.E == 512) {
+        const int waves = M > (M * L.K + 63) / 64 ? M : (M * L.K + 63) / 64;
+        return launch(k_topk_plan<true>, dim3(1), dim3(64 * (waves < 4 ? 4 : waves)), 0, st, L, B, M);
+    }
+    return launch(k_topk_plan<false>, dim3(1), dim3(1024), 0, st, L, B, M);
 }
 
 KernelTimer& kernel_timer() {
@@ -1312,7 +1399,8 @@ hipError_t launch_gate_up(const LayerDev& L, const MoeBufs& B, int M, hipStream_
         if (e != hipSuccess) return e;
         return launch_gu_mfma_g<14, 256, 2, 1>(L, B, M, st);
     }
-    if (L.u8_call) return launch_gu_u8(L, B, M, st);
+    if (L.call_path == kPathU8) return launch_gu_u8(L, B, M, st);
+    if (L.call_path == kPathSeg) return launch_gate_up_pf(L, B, M, st);
     if (moe_uses_fused(L, M)) return launch_gate_down4(L, B, M, nullptr, nullptr, st);
     if (moe_uses_narrow(L, M)) return launch_gate_up4(L, B, M, st);
     const int D = L.p[0].dim;
@@ -1334,7 +1422,11 @@ hipError_t launch_down(const LayerDev& L, const MoeBufs& B, int M, hipStream_t s
         if (e != hipSuccess) return e;
         return launch_down_mfma_g<14, 64, 2, 1>(L, B, M, st);
     }
-    if (L.u8_call) return launch_down_u8(L, B, M, st);
+    if (L.call_path == kPathU8) return launch_down_u8(L, B, M, st);
+    if (L.call_path == kPathSeg) {
+        const hipError_t e = launch_swiglu_pf(L, B, M, st);
+        return e != hipSuccess ? e : launch_down_pf(L, B, M, st);
+    }
     if (moe_uses_fused(L, M)) return hipSuccess;  // (the fused gate/up launch ran the down half)
     if (moe_uses_narrow(L, M)) return launch_down4(L, B, M, st);
     const int D = L.p[2].dim;

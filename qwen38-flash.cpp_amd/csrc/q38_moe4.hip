@@ -783,10 +783,16 @@ bool moe_uses_narrow(const LayerDev& L, int M) {
 
 LayerDev moe_call_dev(const LayerDev& L, int M) {
     LayerDev d = L;
-    d.u8_call = 0;
+    d.call_path = kPathOther;
     if (moe_u8_call(L, M)) {  // the U8 kernels: one plane each, no one-launch layer
-        d.u8_call = 1;
+        d.call_path = kPathU8;
         d.gu_parts = d.d_parts = 1;
+        d.fused_mode = 2;
+        return d;
+    }
+    if (moe_uses_seg_verify(L, M)) {
+        d.call_path = kPathSeg;
+        d.gu_parts = d.d_parts = 2;
         d.fused_mode = 2;
         return d;
     }

@@ -1256,6 +1256,15 @@ int prefill_planes(const LayerDev& L, int M) {
     return 2;
 }
 
+// 5-16 rows: units of mostly one route, so an item costs its gathers whatever the row count, and
+// the 16-row MFMA kernels (a book copy and B staging per item) or, with scale groups, the vector
+// kernels lose. Measured per layer: 13 rows with 64-input groups and an affine shared expert 269
+// -> 80 us (gate/up 161 -> 30, down 77 -> 20), 16 rows with row scales 162 -> 55 us. Up to 4 rows
+// the one-launch kernel is faster.
+bool moe_uses_seg_verify(const LayerDev& L, int M) {
+    return M > 4 && M <= kMaxRows && L.E == 512 && !L.mixed && prefill_planes(L, M) == 2;
+}
+
 template <int NSUB>
 hipError_t launch_gu_seg_t(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
     return launch(L.p[0].ngrp > 1 ? k_gu_seg<NSUB, true> : k_gu_seg<NSUB, false>, dim3(mfma_grid()), dim3(kSegThreads), 0,
@@ -1280,7 +1289,11 @@ hipError_t launch_gate_up_pf(const LayerDev& L, const MoeBufs& B, int M, hipStre
 
 hipError_t launch_swiglu_pf(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
     const int64_t total = static_cast<int64_t>(M * L.K + (L.has_shared ? M : 0)) * L.I;
-    if (prefill_planes(L, M) == 2) return launch(k_swiglu_seg, dim3(2048), dim3(256), 0, st, B, L.I, total);
+    if (prefill_planes(L, M) == 2) {
+        const int64_t blocks = (total + 255) / 256;
+        return launch(k_swiglu_seg, dim3(blocks < 2048 ? static_cast<unsigned>(blocks) : 2048u), dim3(256), 0, st, B, L.I,
+                      total);
+    }
     return launch(k_swiglu_pf, dim3(2048), dim3(256), 0, st, B, total);
 }
 

@@ -88,6 +88,26 @@ def test_sixteen_rows(layer0, q38, orc):
     tol_check(orc, y, wy)
 
 
+@pytest.mark.parametrize("M,k,groups", [(5, 10, None), (9, 10, 64), (16, 16, None), (16, 16, 64), (7, 1, None)])
+def test_wide_verify_rows(gpu, q38, orc, M, k, groups):
+    """5-16 rows on the segmented kernels: the smallest and largest row and route counts, per-row
+    and 64-input scales; the plan with its padding, and row r's bits whatever the call's rows."""
+    geo = dict(top_k=k, gu_group=groups, down_group=groups)
+    L = q38.MoeLayer(gpu, q38.desc(**geo), seed=SEED, layer=4)
+    try:
+        x = orc.rmsnorm(orc.embed(SEED + M, list(range(M)), 2048))
+        y, ex, wt, lg, plan = run_forward(q38, L, L.desc, x)
+        wy, wex, wwt, wlg = orc.moe_layer_synth(oracle_lib.make_desc(**geo), SEED, 4, x)
+        assert np.array_equal(ex, wex) and np.array_equal(wt, wwt)
+        plan_check(orc, plan, ex, 512)
+        n = plan[0]
+        assert (plan[1 + n:1 + M * k] == -1).all() and (plan[1 + M * k + n:2 + 2 * M * k] == M * k).all()
+        tol_check(orc, y, wy)
+        assert np.array_equal(run_forward(q38, L, L.desc, x[:5])[0], y[:5])
+    finally:
+        L.close()
+
+
 def test_repeated_rows_share_experts(layer0, q38, orc):
     """Identical rows route identically; each expert's code rows are applied to both."""
     x1 = orc.normal(orc.key(SEED, 0, 20), 99, 2048, 1.0)
