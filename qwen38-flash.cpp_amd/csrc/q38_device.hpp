@@ -55,6 +55,8 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
     return static_cast<uint16_t>((x & 0x7fffffffu) > 0x7f800000u ? quiet : rounded);
 }
 __device__ __forceinline__ float rbf(float f) { return bf2f(f2bf(f)); }
+// rbf by the conversion instruction (the same nearest-even rounding, two instructions).
+__device__ __forceinline__ float rbf_cvt(float f) { return static_cast<float>(static_cast<__bf16>(f)); }
 __device__ __forceinline__ float h2f(uint16_t h) { return static_cast<float>(__builtin_bit_cast(_Float16, h)); }
 __device__ __forceinline__ uint16_t f2h(float f) { return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f)); }
 

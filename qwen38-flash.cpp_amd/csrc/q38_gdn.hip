@@ -30,7 +30,7 @@ namespace q38 {
 
 namespace {
 
-__device__ __forceinline__ float tbf(float v) { return bf2f(f2bf(v)); }
+__device__ __forceinline__ float tbf(float v) { return rbf_cvt(v); }
 __device__ __forceinline__ float sigmoid_bf(float x) { return tbf(1.0f / (1.0f + expf(-x))); }
 
 // conv + SiLU of row t, channels cb + lane * CPL + i; q / k heads normalised.
@@ -63,8 +63,7 @@ __global__ __launch_bounds__(64) void k_gdn_prework(GdnDev G, GdnBufs B, int S, 
                                              f2bf(cin(t + 1 + j, c));
     }
     if (role < 2) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+        ss = wave_sum_xor(ss);
         const float inv = 1.0f / sqrtf(ss / static_cast<float>(DK) + 1e-6f);
         const float scale = role == 0 ? tbf(1.0f / static_cast<float>(DK)) : tbf(1.0f / sqrtf(static_cast<float>(DK)));
         uint16_t* dst = (role == 0 ? B.q : B.k) + static_cast<size_t>(t) * KW + h * DK + lane * CPL;
@@ -85,10 +84,15 @@ __global__ __launch_bounds__(64) void k_gdn_prework(GdnDev G, GdnBufs B, int S, 
     }
 }
 
-// Lane sum of the 32 lanes of each half-wave in float (xor butterfly 16..1), rounded.
+// Lane sum of the 32 lanes of each half-wave in float (xor butterfly 16..1), rounded. The
+// recurrence is one chain of such sums per row: with LDS permutes for the exchanges, integer
+// roundings and one row of inputs in flight it took 9.9 us at 4 rows, now 6.4.
 __device__ __forceinline__ float half_wave_sum(float v) {
-#pragma unroll
-    for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    v += xor_lane_f<16>(v);
+    v += xor_lane_f<8>(v);
+    v += xor_lane_f<4>(v);
+    v += xor_lane_f<2>(v);
+    v += xor_lane_f<1>(v);
     return tbf(v);
 }
 
@@ -108,8 +112,8 @@ __global__ __launch_bounds__(64) void k_gdn_recur(GdnDev G, GdnBufs B, int S, co
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) st[i] = bf2f(o0[i]);
     }
-    // (row t + 1's inputs are requested before row t's arithmetic; a lane's DK / 32 items of
-    // k, q and the state are one vector access each)
+    // (the inputs of the next four rows are in flight during a row's arithmetic; a lane's DK / 32
+    // items of k, q and the state are one vector access each)
     static_assert(ITEMS == 2 || ITEMS == 4 || ITEMS == 8, "items per lane");
     typedef uint16_t items_t __attribute__((ext_vector_type(ITEMS)));
     struct RowIn {
@@ -125,41 +129,48 @@ __global__ __launch_bounds__(64) void k_gdn_recur(GdnDev G, GdnBufs B, int S, co
         r.g = B.decay[static_cast<size_t>(tt) * HV + hv];
         r.b = B.beta[static_cast<size_t>(tt) * HV + hv];
     };
-    RowIn nxt;
-    load_row(0, nxt);
-    for (int t = 0; t < S; ++t) {
-        const RowIn cur = nxt;
-        load_row(t + 1, nxt);
-        const float g = cur.g, bt = cur.b;
-        float kv[ITEMS], qv[ITEMS];
+    constexpr int kAhead = 4;  // rows in flight
+    RowIn in[kAhead];
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            kv[i] = bf2f(cur.k[i]);
-            qv[i] = bf2f(cur.q[i]);
-        }
-        const float vv = bf2f(cur.v);
-        float acc = 0.0f;
+    for (int u = 0; u < kAhead; ++u) load_row(u, in[u]);
+    for (int t0 = 0; t0 < S; t0 += kAhead) {
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            st[i] = tbf(st[i] * g);
-            acc = tbf(acc + tbf(st[i] * kv[i]));
-        }
-        const float recalled = half_wave_sum(acc);
-        const float delta = tbf(tbf(vv - recalled) * bt);
-        acc = 0.0f;
+        for (int u = 0; u < kAhead; ++u) {
+            const int t = t0 + u;
+            if (t >= S) return;
+            const RowIn cur = in[u];
+            load_row(t + kAhead, in[u]);
+            const float g = cur.g, bt = cur.b;
+            float kv[ITEMS], qv[ITEMS];
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            st[i] = tbf(st[i] + tbf(kv[i] * delta));
-            acc = tbf(acc + tbf(st[i] * qv[i]));
-        }
-        const float y = half_wave_sum(acc);
-        if (sl == 0) B.y[static_cast<size_t>(t) * VW + hv * DV + dv] = f2bf(y);
-        if (ckpt) {
-            typedef uint16_t items_t2 __attribute__((ext_vector_type(ITEMS)));
-            items_t2 o;
+            for (int i = 0; i < ITEMS; ++i) {
+                kv[i] = bf2f(cur.k[i]);
+                qv[i] = bf2f(cur.q[i]);
+            }
+            const float vv = bf2f(cur.v);
+            float acc = 0.0f;
 #pragma unroll
-            for (int i = 0; i < ITEMS; ++i) o[i] = f2bf(st[i]);
-            *reinterpret_cast<items_t2*>(ckpt + static_cast<size_t>(t) * state_elems + rec) = o;
+            for (int i = 0; i < ITEMS; ++i) {
+                st[i] = tbf(st[i] * g);
+                acc = tbf(acc + tbf(st[i] * kv[i]));
+            }
+            const float recalled = half_wave_sum(acc);
+            const float delta = tbf(tbf(vv - recalled) * bt);
+            acc = 0.0f;
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) {
+                st[i] = tbf(st[i] + tbf(kv[i] * delta));
+                acc = tbf(acc + tbf(st[i] * qv[i]));
+            }
+            const float y = half_wave_sum(acc);
+            // (the values are bf16 already: their upper halves)
+            if (sl == 0) B.y[static_cast<size_t>(t) * VW + hv * DV + dv] = static_cast<uint16_t>(__float_as_uint(y) >> 16);
+            if (ckpt) {
+                items_t o;
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i) o[i] = static_cast<uint16_t>(__float_as_uint(st[i]) >> 16);
+                *reinterpret_cast<items_t*>(ckpt + static_cast<size_t>(t) * state_elems + rec) = o;
+            }
         }
     }
 }
@@ -176,8 +187,7 @@ __global__ __launch_bounds__(64) void k_gdn_norm_gate(GdnDev G, GdnBufs B, int S
         y[i] = bf2f(B.y[base + i]);
         ss = fmaf(y[i], y[i], ss);
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    ss = wave_sum_xor(ss);
     const float inv = 1.0f / sqrtf(ss / static_cast<float>(DV) + G.eps);
 #pragma unroll
     for (int i = 0; i < CPL; ++i) {
