@@ -140,7 +140,7 @@ struct LayerDev {
     // H 2048, I 512, per-row scales, no affine shared expert). call_path: the kernels of this
     // verify call (moe_call_dev). kPathU8: those (1-16 rows while they are enabled), one
     // partial-sum plane; kPathSeg: the segmented LDS-codebook kernels of the prefill widths (5-16
-    // rows), two planes, the router storing the fp16 rows chunk-planar; kPathOther: the others.
+    // rows; mixed layers at any), two planes, the router storing the fp16 rows chunk-planar; kPathOther: the others.
     int u8_native, call_path;
 };
 enum { kPathOther = 0, kPathU8 = 1, kPathSeg = 2 };
@@ -279,15 +279,13 @@ hipError_t launch_tile_codes(const uint32_t* codes, int64_t rows, int words, int
 bool moe_uses_mfma(const LayerDev& L);
 // The MFMA layers' geometry, whatever the scale groups.
 bool moe_uses_mfma_geometry(const LayerDev& L);
-// Mixed layer on the MFMA kernels (both banks prepared); the gate/up kernels of both the
-// uniform and the mixed MFMA paths route and build the plan themselves.
-bool moe_mixed_mfma(const LayerDev& L);
+// Whether the call's gate/up kernel routes and builds the plan itself.
 bool moe_plans_in_gate_up(const LayerDev& L, int M);
 // Verify widths of up to 4 rows on the 4x4x4 MFMA kernels (q38_moe4.hip): the MFMA layers,
 // and d8 layers of the same geometry with per-64-input scale groups. They write one partial-
 // sum plane per codebook chunk (gu_parts / d_parts of the call: moe_call_dev).
 bool moe_uses_narrow(const LayerDev& L, int M);
-// Verify widths of 5-16 rows on the segmented kernels (q38_moe_pf.hip).
+// Verify widths on the segmented kernels (q38_moe_pf.hip): 5-16 rows, mixed layers at 1-16.
 bool moe_uses_seg_verify(const LayerDev& L, int M);
 // The layer view of a call of M rows: the partial-sum plane counts of the kernels it takes.
 LayerDev moe_call_dev(const LayerDev& L, int M);

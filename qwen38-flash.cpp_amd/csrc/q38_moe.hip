@@ -495,48 +495,12 @@ __device__ __forceinline__ const uint4* xs_lane(const uint4* xs, int xrow, int z
                                           (active ? xrow : zero_row) * XsLayout<NSUB>::RB + q * XsLayout<NSUB>::QB);
 }
 
-constexpr int kPlanSlots = kMaxRows * kMaxTopK + 1;  // unique-expert slots + the shared one
 
-// Mixed layers: the index of expert e in its bank (even experts and the shared expert E
-// in bank 0, odd experts in bank 1, both at e / 2); uniform layers: e.
-template <int PAR>
-__device__ __forceinline__ int bank_index(int e) { return PAR < 0 ? e : e >> 1; }
-
-// The plan's slots (unique experts ascending, then the shared expert E, which is even)
-// whose expert has parity par, in slot order, into out; returns their count. Every
-// thread calls it; the list is complete after the block barrier inside.
-__device__ __forceinline__ int parity_slots(const int32_t* plan, int nu, int has_shared, int E, int par,
-                                            int32_t* out) {
-    __shared__ int32_t cnt;
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        const int ns = nu + (has_shared ? 1 : 0);
-        int base = 0;
-        for (int u0 = 0; u0 < ns; u0 += 64) {
-            const int u = u0 + lane;
-            const int e = u < nu ? plan[1 + u] : E;
-            const bool take = u < ns && (e & 1) == par;
-            const uint64_t m = __ballot(take);
-            if (take) out[base + __popcll(m & ((1ull << lane) - 1ull))] = u;
-            base += __popcll(m);
-        }
-        if (lane == 0) cnt = base;
-    }
-    __syncthreads();
-    return cnt;
-}
-
-// PAR >= 0 (mixed layers): only the slots whose expert has that parity, with the
-// geometry of that bank (L.pb[proj][PAR], expert index e / 2); the even bank (one codebook
-// chunk) also clears plane 1 of its outputs, so a consumer can add both planes for every
-// route. The even bank's launch routes and publishes the plan; the odd bank's launch,
-// which follows it, reads the plan.
-template <int BITS, int NSUB, int NCHUNK, int PAR = -1>
+template <int BITS, int NSUB, int NCHUNK>
 __global__ __launch_bounds__(kMfmaThreads) void k_gu_mfma(LayerDev L, MoeBufs B, int M) {
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ TopkLds tk;
     __shared__ int32_t plan[kPlanInts];
-    __shared__ int32_t pslots[PAR < 0 ? 1 : kPlanSlots];
     constexpr int KENT = 1 << BITS;
     constexpr int MAXC = gu_mfma_cols(BITS);
     const uint2* book = reinterpret_cast<const uint2*>(lds);       // [KENT] x 4 fp16
@@ -548,29 +512,20 @@ __global__ __launch_bounds__(kMfmaThreads) void k_gu_mfma(LayerDev L, MoeBufs B,
     const int proj = type / NCHUNK, chunk = type % NCHUNK;
     const int per_type = (gridDim.x / (8 * TYPES)) * 8;
     const int idx = (kk / TYPES) * 8 + x8;
-    const ProjDev& P = PAR < 0 ? L.p[proj] : L.pb[proj][PAR < 0 ? 0 : PAR];
+    const ProjDev& P = L.p[proj];
     // waves 0-3 load the codebook chunk while waves 4-7 route; every workgroup derives
     // the same plan and workgroup 0 publishes it
-    if (PAR == 1) {
-        // the odd bank runs right after the even bank's launch, which routed and published
-        // the plan (and the routes) on the same stream
-        for (int i = tid; i < 2 + 4 * M * L.K; i += kMfmaThreads) plan[i] = B.plan[i];
-        fill_book<KENT>(P.book4 + static_cast<size_t>(chunk) * KENT * 4, lds, tid, kMfmaThreads);
-        __syncthreads();
-    } else {
-        // an 8-bit book (2 KiB) is one load per thread of waves 0-3, which then route too
-        constexpr int route_wave0 = KENT <= 256 ? 0 : 4;
-        if (wave < 4) fill_book<KENT>(P.book4 + static_cast<size_t>(chunk) * KENT * 4, lds, tid, 256);
-        topk_plan_block(L, B, M, blockIdx.x == 0, plan, tk, route_wave0);
-        if (blockIdx.x == 0)
-            for (int i = tid; i < 2 + 4 * M * L.K; i += kMfmaThreads) B.plan[i] = plan[i];
-    }
+    // (an 8-bit book, 2 KiB, is one load per thread of waves 0-3, which then route too)
+    constexpr int route_wave0 = KENT <= 256 ? 0 : 4;
+    if (wave < 4) fill_book<KENT>(P.book4 + static_cast<size_t>(chunk) * KENT * 4, lds, tid, 256);
+    topk_plan_block(L, B, M, blockIdx.x == 0, plan, tk, route_wave0);
+    if (blockIdx.x == 0)
+        for (int i = tid; i < 2 + 4 * M * L.K; i += kMfmaThreads) B.plan[i] = plan[i];
     const int H = L.H, I = L.I, K = L.K;
     const int nu = plan[0];
-    const int nslots = PAR < 0 ? nu + (L.has_shared ? 1 : 0) : parity_slots(plan, nu, L.has_shared, L.E, PAR, pslots);
+    const int nslots = nu + (L.has_shared ? 1 : 0);
     const int n_items = nslots * (I / kMfmaRowsPerItem);
     const int tiles = I / kMfmaRowsPerItem;
-    auto slot_of = [&](int item) { return PAR < 0 ? item / tiles : pslots[item / tiles]; };
     float* out = (proj == 0 ? B.g : B.u) + chunk * B.gu_plane;
     const int r16 = lane & 15, q = lane >> 4;
     constexpr int S4 = NSUB / 4;
@@ -589,25 +544,20 @@ __global__ __launch_bounds__(kMfmaThreads) void k_gu_mfma(LayerDev L, MoeBufs B,
     lds_barrier();
     auto code_src = [&](int item) {
         int expert, n, pos0;
-        slot_rows(plan, M, K, L.has_shared, slot_of(item), L.E, &expert, &n, &pos0);
+        slot_rows(plan, M, K, L.has_shared, item / tiles, L.E, &expert, &n, &pos0);
         const size_t rowi =
-            static_cast<size_t>(bank_index<PAR>(expert)) * I + (item % tiles) * kMfmaRowsPerItem + wave * 16 + r16;
+            static_cast<size_t>(expert) * I + (item % tiles) * kMfmaRowsPerItem + wave * 16 + r16;
         return P.codes + rowi * P.words + q * WPL;
     };
-    // Mixed banks: a contiguous range of items, so that consecutive items mostly share a slot
-    // and its staged rows (restaged only when the slot or the pass changes). Uniform layers:
-    // items strided over the workgroups (the shared slot's 16 rows take two passes per tile,
-    // and a contiguous range would put all its tiles on one workgroup).
-    constexpr bool CONTIG = PAR >= 0;
-    const int i0 = CONTIG ? static_cast<int>(static_cast<int64_t>(idx) * n_items / per_type) : idx;
-    const int i1 = CONTIG ? static_cast<int>(static_cast<int64_t>(idx + 1) * n_items / per_type) : n_items;
-    const int istep = CONTIG ? 1 : per_type;
+    // Items strided over the workgroups (the shared slot's 16 rows take two passes per tile, and a
+    // contiguous range would put all its tiles on one workgroup).
+    const int i0 = idx, i1 = n_items, istep = per_type;
     int staged_slot = -1, staged_j0 = -1;
     uint32_t w[WPL + 1], wn[WPL + 1];
     if (i0 < i1) load_lane_words<BITS, NSUB>(code_src(i0), w);
     for (int item = i0; item < i1; item += istep) {
         if (item + istep < i1) load_lane_words<BITS, NSUB>(code_src(item + istep), wn);
-        const int ui = slot_of(item), tile = item % tiles;
+        const int ui = item / tiles, tile = item % tiles;
         int expert, n, pos0;
         slot_rows(plan, M, K, L.has_shared, ui, L.E, &expert, &n, &pos0);
         const bool shared = ui == nu;
@@ -634,9 +584,8 @@ __global__ __launch_bounds__(kMfmaThreads) void k_gu_mfma(LayerDev L, MoeBufs B,
 #pragma unroll
                 for (int rr = 0; rr < 4; ++rr) {
                     const int o = o0 + 4 * q + rr;
-                    const float sc = h2f(P.scales[static_cast<size_t>(bank_index<PAR>(expert)) * I + o]);
+                    const float sc = h2f(P.scales[static_cast<size_t>(expert) * I + o]);
                     out[static_cast<size_t>(pos0 + j0 + r16) * I + o] = sc * acc[rr];
-                    if (PAR >= 0 && NCHUNK == 1) out[B.gu_plane + static_cast<size_t>(pos0 + j0 + r16) * I + o] = 0.0f;
                 }
             }
         }
@@ -647,12 +596,10 @@ __global__ __launch_bounds__(kMfmaThreads) void k_gu_mfma(LayerDev L, MoeBufs B,
 
 constexpr int kDownStageRoutes = 48;  // routes whose SwiGLU rows are staged once (M <= 4 with k = 10)
 
-// PAR >= 0: one bank of a mixed layer, as in k_gu_mfma (the even bank clears plane 1).
-template <int BITS, int NSUB, int NCHUNK, int PAR = -1>
+template <int BITS, int NSUB, int NCHUNK>
 __global__ __launch_bounds__(kMfmaThreads) void k_down_mfma(LayerDev L, MoeBufs B, int M) {
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ int32_t plan[kPlanInts];
-    __shared__ int32_t pslots[PAR < 0 ? 1 : kPlanSlots];
     constexpr int KENT = 1 << BITS;
     const uint2* book = reinterpret_cast<const uint2*>(lds);
     uint4* xs = reinterpret_cast<uint4*>(lds + KENT * 8);   // [routes + 1 zero] SwiGLU rows (XsLayout), 4 fp16 each
@@ -661,7 +608,7 @@ __global__ __launch_bounds__(kMfmaThreads) void k_down_mfma(LayerDev L, MoeBufs 
     const int chunk = kk % NCHUNK;
     const int per_type = (gridDim.x / (8 * NCHUNK)) * 8;
     const int idx = (kk / NCHUNK) * 8 + x8;
-    const ProjDev& P = PAR < 0 ? L.p[2] : L.pb[2][PAR < 0 ? 0 : PAR];
+    const ProjDev& P = L.p[2];
     const int H = L.H, I = L.I, K = L.K;
     const int n_routes = M * K + (L.has_shared ? M : 0);
     for (int i = tid; i < 2 + 4 * M * K; i += kMfmaThreads) plan[i] = B.plan[i];
@@ -692,20 +639,19 @@ __global__ __launch_bounds__(kMfmaThreads) void k_down_mfma(LayerDev L, MoeBufs 
     float* dout = B.d + chunk * B.d_plane;
     const int nu = plan[0];
     const int tiles = H / kMfmaRowsPerItem;
-    const int nslots = PAR < 0 ? nu + (L.has_shared ? 1 : 0) : parity_slots(plan, nu, L.has_shared, L.E, PAR, pslots);
+    const int nslots = nu + (L.has_shared ? 1 : 0);
     const int n_items = nslots * tiles;
-    auto slot_of = [&](int item) { return PAR < 0 ? item / tiles : pslots[item / tiles]; };
     const int r16 = lane & 15, q = lane >> 4;
     constexpr int S4 = NSUB / 4;
     constexpr int WPL = S4 * BITS / 32;
     auto code_src = [&](int item) {
         int expert, n, pos0;
-        slot_rows(plan, M, K, L.has_shared, slot_of(item), L.E, &expert, &n, &pos0);
+        slot_rows(plan, M, K, L.has_shared, item / tiles, L.E, &expert, &n, &pos0);
         const size_t rowi =
-            static_cast<size_t>(bank_index<PAR>(expert)) * H + (item % tiles) * kMfmaRowsPerItem + wave * 16 + r16;
+            static_cast<size_t>(expert) * H + (item % tiles) * kMfmaRowsPerItem + wave * 16 + r16;
         return P.codes + rowi * P.words + q * WPL;
     };
-    // a contiguous range of items (see k_gu_mfma): a slot's routes (all of them when they fit
+    // a contiguous range of items: a slot's routes (all of them when they fit
     // the staging rows) are staged once for its consecutive items
     const int i0 = static_cast<int>(static_cast<int64_t>(idx) * n_items / per_type);
     const int i1 = static_cast<int>(static_cast<int64_t>(idx + 1) * n_items / per_type);
@@ -714,7 +660,7 @@ __global__ __launch_bounds__(kMfmaThreads) void k_down_mfma(LayerDev L, MoeBufs 
     if (i0 < i1) load_lane_words<BITS, NSUB>(code_src(i0), w);
     for (int item = i0; item < i1; ++item) {
         if (item + 1 < i1) load_lane_words<BITS, NSUB>(code_src(item + 1), wn);
-        const int ui = slot_of(item), tile = item % tiles;
+        const int ui = item / tiles, tile = item % tiles;
         int expert, n, pos0;
         slot_rows(plan, M, K, L.has_shared, ui, L.E, &expert, &n, &pos0);
         const int o0 = tile * kMfmaRowsPerItem + wave * 16;
@@ -740,10 +686,9 @@ __global__ __launch_bounds__(kMfmaThreads) void k_down_mfma(LayerDev L, MoeBufs 
 #pragma unroll
                 for (int rr = 0; rr < 4; ++rr) {
                     const int o = o0 + 4 * q + rr;
-                    const float sc = h2f(P.scales[static_cast<size_t>(bank_index<PAR>(expert)) * H + o]);
+                    const float sc = h2f(P.scales[static_cast<size_t>(expert) * H + o]);
                     const size_t at = static_cast<size_t>(route_of_pos(plan, M * K, pos0 + j0 + r16)) * H + o;
                     dout[at] = sc * acc[rr];
-                    if (PAR >= 0 && NCHUNK == 1) B.d[B.d_plane + at] = 0.0f;
                 }
             }
         }
@@ -1257,6 +1202,9 @@ hipError_t launch_route_norm_t(const LayerDev& L, const MoeBufs& B, int M, const
 template <int T, bool NORM>
 hipError_t launch_route_norm_m(const LayerDev& L, const MoeBufs& B, int M, const uint16_t* src, float eps,
                                hipStream_t st) {
+    // (only the kernels of 5-16 rows store the fp16 rows chunk-planar, which the segmented path
+    // reads: mixed layers take it at every width)
+    if (L.call_path == kPathSeg && M <= 8) return launch_route_norm_t<T, NORM, 8>(L, B, M, src, eps, st);
     if (M <= 1) return launch_route_norm_t<T, NORM, 1>(L, B, M, src, eps, st);
     if (M <= 2) return launch_route_norm_t<T, NORM, 2>(L, B, M, src, eps, st);
     if (M <= 4) return launch_route_norm_t<T, NORM, 4>(L, B, M, src, eps, st);
@@ -1269,17 +1217,17 @@ hipError_t launch_route_norm_h(const LayerDev& L, const MoeBufs& B, int M, const
     return norm ? launch_route_norm_m<T, true>(L, B, M, src, eps, st) : launch_route_norm_m<T, false>(L, B, M, src, eps, st);
 }
 
-template <int BITS, int NSUB, int NCHUNK, int PAR = -1>
+template <int BITS, int NSUB, int NCHUNK>
 hipError_t launch_gu_mfma_g(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
     const size_t lds = (size_t{1} << BITS) * 8 + static_cast<size_t>(gu_mfma_cols(BITS) + 1) * XsLayout<NSUB>::RB;
-    if (const hipError_t e = ensure_lds<k_gu_mfma<BITS, NSUB, NCHUNK, PAR>>(lds); e != hipSuccess) return e;
-    return launch(k_gu_mfma<BITS, NSUB, NCHUNK, PAR>, dim3(g_mfma_grid), dim3(kMfmaThreads), lds, st, L, B, M);
+    if (const hipError_t e = ensure_lds<k_gu_mfma<BITS, NSUB, NCHUNK>>(lds); e != hipSuccess) return e;
+    return launch(k_gu_mfma<BITS, NSUB, NCHUNK>, dim3(g_mfma_grid), dim3(kMfmaThreads), lds, st, L, B, M);
 }
-template <int BITS, int NSUB, int NCHUNK, int PAR = -1>
+template <int BITS, int NSUB, int NCHUNK>
 hipError_t launch_down_mfma_g(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
     const size_t lds = (size_t{1} << BITS) * 8 + static_cast<size_t>(kDownStageRoutes + 1) * XsLayout<NSUB>::RB;
-    if (const hipError_t e = ensure_lds<k_down_mfma<BITS, NSUB, NCHUNK, PAR>>(lds); e != hipSuccess) return e;
-    return launch(k_down_mfma<BITS, NSUB, NCHUNK, PAR>, dim3(g_mfma_grid), dim3(kMfmaThreads), lds, st, L, B, M);
+    if (const hipError_t e = ensure_lds<k_down_mfma<BITS, NSUB, NCHUNK>>(lds); e != hipSuccess) return e;
+    return launch(k_down_mfma<BITS, NSUB, NCHUNK>, dim3(g_mfma_grid), dim3(kMfmaThreads), lds, st, L, B, M);
 }
 
 hipError_t launch_gu_u8(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
@@ -1327,17 +1275,9 @@ hipError_t launch_u8_operands(const void* q, int K, int centered, const uint16_t
 
 // Mixed layers run their two banks on the MFMA kernels: H = 2048, I = 512, per-row scales,
 // chunked fp16 codebooks prepared for both banks.
-bool moe_mixed_mfma(const LayerDev& L) {
-    if (!L.mixed || L.H != 2048 || L.I != 512) return false;
-    for (int p = 0; p < 3; ++p)
-        for (int b = 0; b < 2; ++b)
-            if (L.pb[p][b].ngrp != 1 || !L.pb[p][b].book4) return false;
-    return true;
-}
-
 bool moe_plans_in_gate_up(const LayerDev& L, int M) {
     if (L.call_path == kPathSeg) return false;
-    return moe_uses_mfma(L) || moe_mixed_mfma(L) || moe_uses_narrow(L, M);
+    return moe_uses_mfma(L) || moe_uses_narrow(L, M);
 }
 
 bool moe_uses_mfma(const LayerDev& L) {
@@ -1393,12 +1333,7 @@ int mfma_grid() {
 
 hipError_t launch_gate_up(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
     init_grid();
-    if (L.mixed) {  // the two banks on the MFMA kernels: even experts d4/8-bit, odd d8/14-bit
-        if (!moe_mixed_mfma(L)) return hipErrorInvalidValue;
-        const hipError_t e = launch_gu_mfma_g<8, 512, 1, 0>(L, B, M, st);
-        if (e != hipSuccess) return e;
-        return launch_gu_mfma_g<14, 256, 2, 1>(L, B, M, st);
-    }
+    if (L.mixed && L.call_path != kPathSeg) return hipErrorInvalidValue;
     if (L.call_path == kPathU8) return launch_gu_u8(L, B, M, st);
     if (L.call_path == kPathSeg) return launch_gate_up_pf(L, B, M, st);
     if (moe_uses_fused(L, M)) return launch_gate_down4(L, B, M, nullptr, nullptr, st);
@@ -1416,12 +1351,7 @@ hipError_t launch_gate_up(const LayerDev& L, const MoeBufs& B, int M, hipStream_
 
 hipError_t launch_down(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
     init_grid();
-    if (L.mixed) {
-        if (!moe_mixed_mfma(L)) return hipErrorInvalidValue;
-        const hipError_t e = launch_down_mfma_g<8, 128, 1, 0>(L, B, M, st);
-        if (e != hipSuccess) return e;
-        return launch_down_mfma_g<14, 64, 2, 1>(L, B, M, st);
-    }
+    if (L.mixed && L.call_path != kPathSeg) return hipErrorInvalidValue;
     if (L.call_path == kPathU8) return launch_down_u8(L, B, M, st);
     if (L.call_path == kPathSeg) {
         const hipError_t e = launch_swiglu_pf(L, B, M, st);

@@ -519,8 +519,10 @@ struct SegTab {
 __device__ __forceinline__ void seg_wait_vm() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // ustart[s] = the first unit of slot s (ustart[ns] = the unit count): slot s has
-// ceil(n_s / 16) units. One wave, 64 slots per step (inclusive scan by shuffles).
-__device__ __forceinline__ void seg_unit_scan(const int32_t* plan, int M, int K, int has_shared, int32_t* ustart) {
+// ceil(n_s / 16) units, or none where its expert is not of parity par (mixed layers; par < 0:
+// every slot). One wave, 64 slots per step (inclusive scan by shuffles).
+template <int PAR>
+__device__ __forceinline__ void seg_unit_scan(const int32_t* plan, int M, int K, int has_shared, int E, int32_t* ustart) {
     const int lane = threadIdx.x & 63;
     const int nu = plan[0], ns = nu + (has_shared ? 1 : 0), MK = M * K;
     int base = 0;
@@ -529,6 +531,7 @@ __device__ __forceinline__ void seg_unit_scan(const int32_t* plan, int M, int K,
         int n = 0;
         if (s < nu) n = plan[1 + MK + s + 1] - plan[1 + MK + s];
         else if (s < ns) n = M;
+        if (PAR >= 0 && ((s < nu ? plan[1 + s] : E) & 1) != PAR) n = 0;
         int v = (n + kSegRoutes - 1) / kSegRoutes;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -541,7 +544,7 @@ __device__ __forceinline__ void seg_unit_scan(const int32_t* plan, int M, int K,
     if (lane == 0) ustart[0] = 0;
 }
 
-// Slot of unit u: the last s with ustart[s] <= u (every slot has at least one unit).
+// Slot of unit u: the last s with ustart[s] <= u.
 __device__ __forceinline__ int seg_slot(const int32_t* ustart, int ns, int u) {
     int lo = 0, hi = ns;
     while (hi - lo > 1) {
@@ -553,7 +556,8 @@ __device__ __forceinline__ int seg_slot(const int32_t* ustart, int ns, int u) {
 }
 
 // The table of units [u0, u0 + nt) (every thread of the workgroup; ustart published).
-template <bool DOWN>
+// (mixed layers: the expert's index in its bank)
+template <bool DOWN, int PAR>
 __device__ __forceinline__ void seg_build_tab(const int32_t* plan, int M, int K, int has_shared, int E, int ns,
                                               int u0, int nt, SegTab& T) {
     const int MK = M * K, nu = plan[0];
@@ -564,7 +568,7 @@ __device__ __forceinline__ void seg_build_tab(const int32_t* plan, int M, int K,
         int expert, n, pos0;
         slot_rows(plan, M, K, has_shared, s, E, &expert, &n, &pos0);
         const int j0 = (u - T.ustart[s]) * kSegRoutes, j = j0 + l;
-        if (l == 0) T.unit[k] = make_int4(expert, n, pos0, j0);
+        if (l == 0) T.unit[k] = make_int4(PAR < 0 ? expert : expert >> 1, n, pos0, j0);
         int r = -1;
         if (j < n) r = DOWN ? route_of_pos(plan, MK, pos0 + j) : route_row(plan, M, K, pos0, j, s == nu);
         T.row[k][l] = r;
@@ -629,19 +633,42 @@ __device__ __forceinline__ uint32_t code14_x8(const uint32_t* w, int q) {
     return v & (((1u << 14) - 1u) << 3);
 }
 
+// d4/8-bit codes (the even bank of mixed layers): subvectors 2 t and 2 t + 1 of four dims are the
+// chunks of an 8-dim subvector t, so chunk c of the layer takes every second byte and the inputs
+// keep the chunk-planar layout. A lane's span of SPL subvectors t is 2 SPL / 32 blocks of 8 words;
+// each word, shifted by 8 c, holds the codes of a pair of t in bytes 0 and 2.
+template <int SPL>
+__device__ __forceinline__ void seg_load_bytes(const uint32_t* codes_t, int blocks, size_t tile64, int rr, int span,
+                                               uint32_t (&w)[SPL / 2]) {
+    const uint32_t* base = codes_t + (tile64 * blocks + span * (SPL / 16)) * (8 * 64) + rr * 4;
+#pragma unroll
+    for (int c = 0; c < SPL / 8; ++c) {  // (two chunks of 4 words per block)
+        const uint4 v = *reinterpret_cast<const uint4*>(base + c * 256);
+        w[4 * c] = v.x; w[4 * c + 1] = v.y; w[4 * c + 2] = v.z; w[4 * c + 3] = v.w;
+    }
+}
+
+// The LDS byte offsets of the entries of subvectors 2 t, 2 t + 1.
+template <int BITS>
+__device__ __forceinline__ uint2 seg_offsets(const uint32_t* w, int t) {
+    if constexpr (BITS == 14) return make_uint2(code14_x8(w, 2 * t), code14_x8(w, 2 * t + 1));
+    else return make_uint2((w[t] << 3) & 0x7F8u, (w[t] >> 13) & 0x7F8u);
+}
+
 // Two 16-row tiles of one item: acc[i] += A(rows of w[i]) x B over NB16 16-byte B words (two
 // subvectors each). MFMA m (step m / 2, tile m % 2) uses the gathers issued LA MFMAs
 // earlier: scheduling barriers keep that order (left alone, the scheduler waits for each
 // MFMA's two gathers right before it, and the LDS latency is exposed on every step).
-template <int NB16, int NW>
+template <int BITS, int NB16, int NW>
 __device__ __forceinline__ void seg_mfma(const uint32_t (&w)[2][NW], const uint4 (&bx)[NB16],
                                          const unsigned char* book, f4_t (&acc)[2]) {
     constexpr int NM = 2 * NB16, LA = 4;
     uint4 a[NM];
     auto gather = [&](int m) {
         const int t = m >> 1, i = m & 1;
-        const uint2 a0 = *reinterpret_cast<const uint2*>(book + code14_x8(w[i], 2 * t));
-        const uint2 a1 = *reinterpret_cast<const uint2*>(book + code14_x8(w[i], 2 * t + 1));
+        const uint2 o = seg_offsets<BITS>(w[i], t);
+        const uint2 a0 = *reinterpret_cast<const uint2*>(book + o.x);
+        const uint2 a1 = *reinterpret_cast<const uint2*>(book + o.y);
         a[m] = make_uint4(a0.x, a0.y, a1.x, a1.y);
     };
 #pragma unroll
@@ -787,38 +814,35 @@ __device__ __forceinline__ void seg_range(int n_items, int per_type, int idx, in
 // four K parts would not fit in LDS beside the 128 KiB codebook chunk). Output rows of an item:
 // TR = 32 * RG rows of I; chunk `chunk` of projection `proj` per workgroup type. B = rows of
 // the chunk-planar fp16 inputs ([2][M][H / 2]).
-// G8: one scale per 64 inputs (ngrp = H / 64) instead of one per output row.
-template <int NSUB, bool G8>
-__global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, int M) {
-    constexpr int KP = NSUB / 128, RG = 8 / KP, TR = 32 * RG, KS = NSUB / 32;
-    static_assert(NSUB % 128 == 0 && KP * RG == 8, "8 waves = K parts x row groups");
+// G8: one scale per 64 inputs (ngrp = H / 64) instead of one per output row. PAR >= 0: the bank of
+// a mixed layer (BITS 8: the even one).
+template <int NSUB>
+struct GuSegLds {
+    static constexpr int KP = NSUB / 128, RG = 8 / KP, RED = 2 * (KP - 1) * RG * 2 * 64;
     // One static LDS block (the codebook chunk at offset 0, known when compiling, so a gather's
     // address is its code offset alone), the K-part partial sums ([2][KP - 1][RG][2][64]) and
     // the unit table.
-    constexpr int RED = 2 * (KP - 1) * RG * 2 * 64;
-    struct Lds {
-        uint2 book[kSegKent];
-        f4_t red[RED > 0 ? RED : 1];
-        SegTab T;
-    };
-    __shared__ Lds S;
+    uint2 book[kSegKent];
+    f4_t red[RED > 0 ? RED : 1];
+    SegTab T;
+};
+template <int NSUB, bool G8, int BITS, int PAR>
+__device__ __forceinline__ void gu_seg_body(const LayerDev& L, const MoeBufs& B, int M, const ProjDev& P, int proj,
+                                            int chunk, int per_type, int idx, GuSegLds<NSUB>& S) {
+    constexpr int KP = NSUB / 128, RG = 8 / KP, TR = 32 * RG, KS = NSUB / 32, KENT = 1 << BITS;
+    constexpr int NW = BITS == 14 ? 14 : 16;  // words of a lane's 32-subvector span
+    static_assert(NSUB % 128 == 0 && KP * RG == 8, "8 waves = K parts x row groups");
     unsigned char* lds = reinterpret_cast<unsigned char*>(S.book);
     const unsigned char* book = lds;
     f4_t* red = S.red;
     SegTab& T = S.T;
-    touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kh = wave % KP, rg = wave / KP;
     const int r16 = lane & 15, q = lane >> 4;
-    const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
-    const int type = kk & 3, proj = type >> 1, chunk = type & 1;
-    const int per_type = (gridDim.x / 32) * 8;
-    const int idx = (kk >> 2) * 8 + x8;  // the chunk-0 and chunk-1 workgroups of an index share an XCD
-    const ProjDev& P = L.p[proj];
     const int H = L.H, I = L.I, K = L.K, E = L.E, hs = L.has_shared;
     const int32_t* plan = B.plan;
-    if (wave == 0) seg_unit_scan(plan, M, K, hs, T.ustart);
-    else dma_book<kSegKent>(P.book4 + static_cast<size_t>(chunk) * kSegKent * 4, lds, wave - 1, 7);
+    if (wave == 0) seg_unit_scan<PAR>(plan, M, K, hs, E, T.ustart);
+    else dma_book<KENT>(P.book4 + (BITS == 14 ? static_cast<size_t>(chunk) * KENT * 4 : 0), lds, wave - 1, 7);
     lds_barrier_dma_pending();  // ustart published; the codebook copy still in flight
     const int ns = plan[0] + (hs ? 1 : 0);
     const int tiles = I / TR;
@@ -829,7 +853,7 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
         return;
     }
     const int u0 = i0 / tiles;
-    seg_build_tab<false>(plan, M, K, hs, E, ns, u0, (i1 - 1) / tiles - u0 + 1, T);
+    seg_build_tab<false, PAR>(plan, M, K, hs, E, ns, u0, (i1 - 1) / tiles - u0 + 1, T);
     seg_wait_vm();
     lds_barrier();
     float* out = (proj == 0 ? B.g : B.u) + chunk * B.gu_plane;
@@ -849,12 +873,14 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
             for (int i = 0; i < 16; ++i) bx[i] = make_uint4(0u, 0u, 0u, 0u);
         }
     };
-    auto load_codes = [&](int expert, int tile, uint32_t (&w)[2][14]) {
+    auto load_codes = [&](int expert, int tile, uint32_t (&w)[2][NW]) {
         const size_t row0 = static_cast<size_t>(expert) * I + tile * TR + rg * 32;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-            seg_load_codes<32>(P.codes_t, KS, row0 >> 6, static_cast<int>(row0 & 63) + 16 * i + r16, kh * 4 + q, 0,
-                               w[i]);
+        for (int i = 0; i < 2; ++i) {
+            const int rr = static_cast<int>(row0 & 63) + 16 * i + r16;
+            if constexpr (BITS == 14) seg_load_codes<32>(P.codes_t, KS, row0 >> 6, rr, kh * 4 + q, 0, w[i]);
+            else seg_load_bytes<32>(P.codes_t, 2 * KS, row0 >> 6, rr, kh * 4 + q, w[i]);
+        }
     };
     if constexpr (G8) {
         auto load_scales = [&](int expert, int tile, uint32_t (&sc)[2][8]) {
@@ -924,7 +950,7 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
     load_b(0, bx);
     // (k, tile): the current item's unit (table index) and tile, advanced without divisions
     int k = 0, tile = i0 - u0 * tiles;
-    auto body = [&](int item, const uint32_t (&w)[2][14], uint32_t (&wn)[2][14]) {
+    auto body = [&](int item, uint32_t (&w)[2][NW], uint32_t (&wn)[2][NW]) {
         const int4 un = T.unit[k];  // expert, n, pos0, j0
         const int o0 = tile * TR + rg * 32 + 4 * q;
         // loads in the order they are needed: this item's row scales, the next unit's B
@@ -937,7 +963,12 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
         const bool new_unit = !last && tile + 1 == tiles;
         load_codes(new_unit ? T.unit[k + 1].x : un.x, last ? tile : new_unit ? 0 : tile + 1, wn);
         f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
-        seg_mfma<16, 14>(w, bx, book, acc);
+        if constexpr (BITS == 8)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int v = 0; v < NW; ++v) w[i][v] >>= 8 * chunk;
+        seg_mfma<BITS, 16, NW>(w, bx, book, acc);
         // the next unit's B operand replaces this one as soon as the MFMAs have read it (a
         // second register set would not fit), in flight through the reduction and stores
         if (new_unit) load_b(k + 1, bx);
@@ -967,7 +998,7 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
             ++tile;
         }
     };
-    uint32_t wa[2][14], wb[2][14];
+    uint32_t wa[2][NW], wb[2][NW];
     load_codes(T.unit[0].x, tile, wa);
     for (int item = i0; item < i1; item += 2) {
         body(item, wa, wb);
@@ -975,37 +1006,52 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
     }
 }
 
+template <int NSUB, bool G8>
+__global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, int M) {
+    __shared__ GuSegLds<NSUB> S;
+    touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
+    const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
+    const int type = kk & 3, proj = type >> 1, chunk = type & 1;
+    // (the chunk-0 and chunk-1 workgroups of an index share an XCD)
+    gu_seg_body<NSUB, G8, 14, -1>(L, B, M, L.p[proj], proj, chunk, (gridDim.x / 32) * 8, (kk >> 2) * 8 + x8, S);
+}
+// Both banks of a mixed layer in one launch: workgroup types bank x projection x chunk, half of
+// the workgroups each bank (an item costs its gathers, the same number in both). 16 rows: 32 us,
+// and 19 us for the down kernel, against 41 + 26 and 28 + 24 us of 16-row kernels that ran one
+// bank after the other, staged their operand rows and, for the d4 bank, cleared the second plane.
+__global__ __launch_bounds__(kSegThreads) void k_gu_seg_mixed(LayerDev L, MoeBufs B, int M) {
+    __shared__ GuSegLds<256> S;
+    touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
+    const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
+    const int type = kk & 7, proj = (type >> 1) & 1, chunk = type & 1;
+    const int per_type = (gridDim.x / 64) * 8, idx = (kk >> 3) * 8 + x8;
+    if (type & 4) gu_seg_body<256, false, 14, 1>(L, B, M, L.pb[proj][1], proj, chunk, per_type, idx, S);
+    else gu_seg_body<256, false, 8, 0>(L, B, M, L.pb[proj][0], proj, chunk, per_type, idx, S);
+}
+
 // Down (NSUB = I / 8 subvectors per row: 64 or 128; SPL = NSUB / 4 per lane quarter, 16 =
 // half a code block). One K part: wave rg owns rows 32 rg .. + 31 of a TR = 256-row tile of
 // H. B = the pass's SwiGLU rows (chunk-planar fp16 at sorted positions); outputs at the
 // route index.
-template <int NSUB, bool G8>
-__global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, int M) {
-    constexpr int SPL = NSUB / 4, TR = 256, KS = NSUB / 32;
+struct DnSegLds {  // one static LDS block, as for gate/up
+    uint2 book[kSegKent];
+    SegTab T;
+};
+template <int NSUB, bool G8, int BITS, int PAR>
+__device__ __forceinline__ void dn_seg_body(const LayerDev& L, const MoeBufs& B, int M, const ProjDev& P, int chunk,
+                                            int per_type, int idx, DnSegLds& S) {
+    constexpr int SPL = NSUB / 4, TR = 256, KS = NSUB / 32, KENT = 1 << BITS;
     static_assert(SPL == 16 || SPL == 32, "16-code or 32-code lane spans");
-    constexpr int NW = SPL == 32 ? 14 : 7, NB = SPL / 2;
-    // one static LDS block: the codebook chunk at offset 0 (a gather's address is its code
-    // offset alone), then the unit table
-    struct Lds {
-        uint2 book[kSegKent];
-        SegTab T;
-    };
-    __shared__ Lds S;
+    constexpr int NB = SPL / 2, NW = BITS == 8 ? SPL / 2 : SPL == 32 ? 14 : 7;
     unsigned char* lds = reinterpret_cast<unsigned char*>(S.book);
     const unsigned char* book = lds;
     SegTab& T = S.T;
-    touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
     const int tid = threadIdx.x, lane = tid & 63, rg = tid >> 6;
     const int r16 = lane & 15, q = lane >> 4;
-    const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
-    const int chunk = kk & 1;
-    const int per_type = (gridDim.x / 16) * 8;
-    const int idx = (kk >> 1) * 8 + x8;
-    const ProjDev& P = L.p[2];
     const int H = L.H, I = L.I, K = L.K, E = L.E, hs = L.has_shared;
     const int32_t* plan = B.plan;
-    if (rg == 0) seg_unit_scan(plan, M, K, hs, T.ustart);
-    else dma_book<kSegKent>(P.book4 + static_cast<size_t>(chunk) * kSegKent * 4, lds, rg - 1, 7);
+    if (rg == 0) seg_unit_scan<PAR>(plan, M, K, hs, E, T.ustart);
+    else dma_book<KENT>(P.book4 + (BITS == 14 ? static_cast<size_t>(chunk) * KENT * 4 : 0), lds, rg - 1, 7);
     lds_barrier_dma_pending();
     const int ns = plan[0] + (hs ? 1 : 0);
     const int tiles = H / TR;
@@ -1016,7 +1062,7 @@ __global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, i
         return;
     }
     const int u0 = i0 / tiles;
-    seg_build_tab<true>(plan, M, K, hs, E, ns, u0, (i1 - 1) / tiles - u0 + 1, T);
+    seg_build_tab<true, PAR>(plan, M, K, hs, E, ns, u0, (i1 - 1) / tiles - u0 + 1, T);
     seg_wait_vm();
     lds_barrier();
     float* dout = B.d + chunk * B.d_plane;
@@ -1042,9 +1088,11 @@ __global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, i
     auto load_codes = [&](int expert, int tile, uint32_t (&w)[2][NW]) {
         const size_t row0 = static_cast<size_t>(expert) * H + tile * TR + rg * 32;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-            seg_load_codes<SPL>(P.codes_t, KS, row0 >> 6, static_cast<int>(row0 & 63) + 16 * i + r16, blk, half,
-                                w[i]);
+        for (int i = 0; i < 2; ++i) {
+            const int rr = static_cast<int>(row0 & 63) + 16 * i + r16;
+            if constexpr (BITS == 14) seg_load_codes<SPL>(P.codes_t, KS, row0 >> 6, rr, blk, half, w[i]);
+            else seg_load_bytes<SPL>(P.codes_t, 2 * KS, row0 >> 6, rr, q, w[i]);
+        }
     };
     if constexpr (G8) {
         auto load_scales = [&](int expert, int tile, uint32_t (&sc)[2][NB / 2]) {
@@ -1103,7 +1151,7 @@ __global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, i
     uint4 bx[NB];
     load_b(0, bx);
     int k = 0, tile = i0 - u0 * tiles;
-    auto body = [&](int item, const uint32_t (&w)[2][NW], uint32_t (&wn)[2][NW]) {
+    auto body = [&](int item, uint32_t (&w)[2][NW], uint32_t (&wn)[2][NW]) {
         const int expert = T.unit[k].x;
         const int rt = T.row[k][r16];  // route index of the lane's route (-1: none)
         const int o0 = tile * TR + rg * 32 + 4 * q;
@@ -1114,7 +1162,12 @@ __global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, i
         const bool new_unit = !last && tile + 1 == tiles;
         load_codes(new_unit ? T.unit[k + 1].x : expert, last ? tile : new_unit ? 0 : tile + 1, wn);
         f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
-        seg_mfma<NB, NW>(w, bx, book, acc);
+        if constexpr (BITS == 8)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int v = 0; v < NW; ++v) w[i][v] >>= 8 * chunk;
+        seg_mfma<BITS, NB, NW>(w, bx, book, acc);
         if (new_unit) load_b(k + 1, bx);
         if (rt >= 0)
 #pragma unroll
@@ -1133,6 +1186,22 @@ __global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, i
         body(item, wa, wb);
         if (item + 1 < i1) body(item + 1, wb, wa);
     }
+}
+
+template <int NSUB, bool G8>
+__global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, int M) {
+    __shared__ DnSegLds S;
+    touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
+    const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
+    dn_seg_body<NSUB, G8, 14, -1>(L, B, M, L.p[2], kk & 1, (gridDim.x / 16) * 8, (kk >> 1) * 8 + x8, S);
+}
+__global__ __launch_bounds__(kSegThreads) void k_dn_seg_mixed(LayerDev L, MoeBufs B, int M) {
+    __shared__ DnSegLds S;
+    touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
+    const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
+    const int chunk = kk & 1, per_type = (gridDim.x / 32) * 8, idx = (kk >> 2) * 8 + x8;
+    if (kk & 2) dn_seg_body<64, false, 14, 1>(L, B, M, L.pb[2][1], chunk, per_type, idx, S);
+    else dn_seg_body<64, false, 8, 0>(L, B, M, L.pb[2][0], chunk, per_type, idx, S);
 }
 
 // SwiGLU of every route, the two chunk planes of g and u added; the output is chunk-planar
@@ -1256,13 +1325,24 @@ int prefill_planes(const LayerDev& L, int M) {
     return 2;
 }
 
+// Mixed layers (verify widths; H 2048, I 512, row scales): both banks' codes tiled and books in
+// chunks.
+static bool moe_mixed_seg(const LayerDev& L) {
+    if (!L.mixed || L.H != 2048 || L.I != 512) return false;
+    for (int p = 0; p < 3; ++p)
+        for (int b = 0; b < 2; ++b)
+            if (L.pb[p][b].ngrp != 1 || !L.pb[p][b].book4 || !L.pb[p][b].codes_t) return false;
+    return true;
+}
+
 // 5-16 rows: units of mostly one route, so an item costs its gathers whatever the row count, and
 // the 16-row MFMA kernels (a book copy and B staging per item) or, with scale groups, the vector
 // kernels lose. Measured per layer: 13 rows with 64-input groups and an affine shared expert 269
 // -> 80 us (gate/up 161 -> 30, down 77 -> 20), 16 rows with row scales 162 -> 55 us. Up to 4 rows
 // the one-launch kernel is faster.
 bool moe_uses_seg_verify(const LayerDev& L, int M) {
-    return M > 4 && M <= kMaxRows && L.E == 512 && !L.mixed && prefill_planes(L, M) == 2;
+    if (L.mixed) return moe_mixed_seg(L);
+    return M > 4 && M <= kMaxRows && L.E == 512 && prefill_planes(L, M) == 2;
 }
 
 template <int NSUB>
@@ -1277,6 +1357,10 @@ hipError_t launch_dn_seg_t(const LayerDev& L, const MoeBufs& B, int M, hipStream
 }
 
 hipError_t launch_gate_up_pf(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
+    if (L.mixed) {  // (eight workgroup types of 8 XCDs)
+        if (mfma_grid() < 64) return hipErrorInvalidValue;
+        return launch(k_gu_seg_mixed, dim3(mfma_grid() / 64 * 64), dim3(kSegThreads), 0, st, L, B, M);
+    }
     if (prefill_planes(L, M) == 2) {
         switch (L.H / 8) {
             case 128: return launch_gu_seg_t<128>(L, B, M, st);
@@ -1289,7 +1373,7 @@ hipError_t launch_gate_up_pf(const LayerDev& L, const MoeBufs& B, int M, hipStre
 
 hipError_t launch_swiglu_pf(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
     const int64_t total = static_cast<int64_t>(M * L.K + (L.has_shared ? M : 0)) * L.I;
-    if (prefill_planes(L, M) == 2) {
+    if (L.mixed || prefill_planes(L, M) == 2) {
         const int64_t blocks = (total + 255) / 256;
         return launch(k_swiglu_seg, dim3(blocks < 2048 ? static_cast<unsigned>(blocks) : 2048u), dim3(256), 0, st, B, L.I,
                       total);
@@ -1298,6 +1382,7 @@ hipError_t launch_swiglu_pf(const LayerDev& L, const MoeBufs& B, int M, hipStrea
 }
 
 hipError_t launch_down_pf(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
+    if (L.mixed) return launch(k_dn_seg_mixed, dim3(mfma_grid()), dim3(kSegThreads), 0, st, L, B, M);
     if (prefill_planes(L, M) == 2) {
         if (L.I / 8 == 64) return launch_dn_seg_t<64>(L, B, M, st);
         if (L.I / 8 == 128) return launch_dn_seg_t<128>(L, B, M, st);
