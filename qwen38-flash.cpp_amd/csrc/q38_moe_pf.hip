@@ -1309,7 +1309,7 @@ static int64_t seg_units_per_wg(const LayerDev& L, int M, int tiles, int per_typ
 
 int prefill_planes(const LayerDev& L, int M) {
     for (int p = 0; p < 3; ++p) {
-        if (!L.p[p].book4 || !L.p[p].codes_t) return 1;
+        if (L.p[p].dim != 8 || L.p[p].bits != 14 || !L.p[p].book4 || !L.p[p].codes_t) return 1;
         // one scale per row or per 64 inputs
         if (L.p[p].ngrp != 1 && L.p[p].ngrp * 64 != (p < 2 ? L.H : L.I)) return 1;
     }

@@ -108,6 +108,23 @@ def test_wide_verify_rows(gpu, q38, orc, M, k, groups):
         L.close()
 
 
+@pytest.mark.parametrize("geo", [dict(gu=(4, 8), down=(4, 8)), dict(gu=(4, 8)), dict(down=(4, 8))])
+@pytest.mark.parametrize("M", [5, 16])
+def test_wide_verify_rows_byte_codes(gpu, q38, orc, geo, M):
+    """5-16 rows of 512-expert layers with d4/8-bit projections: not the segmented kernels, which
+    read 14-bit codes."""
+    L = q38.MoeLayer(gpu, q38.desc(**geo), seed=SEED, layer=5)
+    try:
+        x = orc.normal(orc.key(SEED, 5, 20), 23 * M, M * 2048, 1.0).reshape(M, 2048)
+        y, ex, wt, lg, plan = run_forward(q38, L, L.desc, x)
+        wy, wex, wwt, wlg = orc.moe_layer_synth(oracle_lib.make_desc(**geo), SEED, 5, x)
+        assert np.array_equal(ex, wex) and np.array_equal(wt, wwt)
+        plan_check(orc, plan, ex, 512)
+        tol_check(orc, y, wy)
+    finally:
+        L.close()
+
+
 def test_repeated_rows_share_experts(layer0, q38, orc):
     """Identical rows route identically; each expert's code rows are applied to both."""
     x1 = orc.normal(orc.key(SEED, 0, 20), 99, 2048, 1.0)
