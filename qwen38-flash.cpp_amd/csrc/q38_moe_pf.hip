@@ -1,7 +1,7 @@
 // q38_moe_pf.hip — prefill-width sparse MoE (R1-R3, R9): 17..2048 rows per call, the
 // SparseMoe::forward_prefill_impl segmented path (src/sparse_moe.cpp:2199-2624).
 //
-//   k_logits_rows  router logits, NE router rows per workgroup held in registers across
+//   k_logits_rows  router logits, NE router rows per wave held in registers across
 //                  the workgroup's request rows (the per-lane summation contract of the
 //                  verify router), and the shared expert's gate
 //   k_topk_rows    softmax + top-k of every row (one wave per row, R2)
@@ -29,12 +29,16 @@ typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 
 // ============================================================== router (R1)
-// Workgroup (gx, gy): routed router rows [NE gx, NE gx + NE) against request rows
-// [rpw gy, rpw gy + rpw), wave w taking rows rpw gy + w, + 8, ... Lane l accumulates
-// x*w over the columns 512t + 8l + j (t outer, j inner) with fmaf, then the xor butterfly
-// and BF16 rounding: the logits equal the verify router's bit for bit. The launch sizes rpw
-// so that the grid is resident at once (one pass of workgroups per CU slot, no partial
-// second pass).
+// Workgroup (gx, gy): request rows [rpw gy, rpw gy + rpw), wave w the NE routed router rows from
+// NE (8 gx + w), held in registers. The eight waves walk the same request rows, so a row comes
+// from the L2 once per workgroup, and the rows' copies and gates are dealt over all waves. Lane l
+// accumulates x*w over the columns 512t + 8l + j (t outer, j inner) with fmaf, then the xor
+// butterfly and BF16 rounding: the logits equal the verify router's bit for bit. The launch sizes
+// rpw so that the grid is resident at once (one pass of workgroups per CU slot, no partial
+// second pass). Bound by the FP32 FMAs and the conversions of x: 2,048 rows x 512 experts 158 -> 98
+// us, 512 rows 43 -> 31 us, against waves that shared the router rows and took every eighth
+// request row (then every wave read other rows, 1 GiB through the L2s at 2,048, and the first
+// column of workgroups wrote all the copies).
 // planar: the fp16 copy of x is stored chunk-planar ([2][M][H / 2]: dims 4c..4c+3 of every
 // subvector in plane c), the layout the LDS-codebook gate/up kernel reads its B operand from.
 constexpr int kLogitsWaves = 8;
@@ -43,8 +47,9 @@ template <int T, int NE>
 __global__ __launch_bounds__(64 * kLogitsWaves) void k_logits_rows(LayerDev L, MoeBufs B, int M, const uint16_t* __restrict__ x,
                                                      int planar, int rpw) {
     constexpr int H = 512 * T;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int e0 = blockIdx.x * NE;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int job = static_cast<int>(blockIdx.x) * kLogitsWaves + wave, jobs = static_cast<int>(gridDim.x) * kLogitsWaves;
+    const int e0 = job * NE;
     const int nr = L.E;
     uint4 wv[NE][T];
 #pragma unroll
@@ -54,7 +59,7 @@ __global__ __launch_bounds__(64 * kLogitsWaves) void k_logits_rows(LayerDev L, M
 #pragma unroll
         for (int t = 0; t < T; ++t) wv[n][t] = *reinterpret_cast<const uint4*>(w + 512 * t + 8 * lane);
     }
-    const bool store_x = blockIdx.x == 0 && x != B.x;
+    const bool store_x = x != B.x;
     const int rb = static_cast<int>(blockIdx.y) * rpw;
     const int r1 = rb + rpw < M ? rb + rpw : M;
     if (rb >= r1) return;
@@ -65,8 +70,8 @@ __global__ __launch_bounds__(64 * kLogitsWaves) void k_logits_rows(LayerDev L, M
     // the request rows two and one steps ahead are in flight while a row's dot products run
     // (past the end the last row again: always in bounds)
     uint4 xa[T], xb[T];
-    load_row(rb + wave < r1 ? rb + wave : r1 - 1, xa);
-    load_row(rb + wave + kLogitsWaves < r1 ? rb + wave + kLogitsWaves : r1 - 1, xb);
+    load_row(rb, xa);
+    load_row(rb + 1 < r1 ? rb + 1 : r1 - 1, xb);
     // the router bias of the lane's logits (loop-invariant: loaded once, so that no load in the
     // loop waits behind the prefetches)
     float rbias[scatter_slots<NE>()];
@@ -75,14 +80,14 @@ __global__ __launch_bounds__(64 * kLogitsWaves) void k_logits_rows(LayerDev L, M
         const int e = e0 + scatter_value<NE>(s, lane >> 4);
         rbias[s] = L.rbias ? L.rbias[e < nr ? e : nr - 1] : 0.0f;
     }
-    // The shared expert's gate row (w_sg), spread over the grid's columns: wave 0 of column gx
-    // takes request rows rb + gx, rb + gx + gridDim.x, ... of its range, with the same lane
-    // contract; sgate = T(sigmoid(T(logit))).
-    if (L.has_shared && wave == 0) {
+    // The shared expert's gate row (w_sg), spread over the grid's columns: wave `job` of `jobs` takes
+    // request rows rb + job, rb + job + jobs, ... of its range, with the same lane contract;
+    // sgate = T(sigmoid(T(logit))).
+    if (L.has_shared && rb + job < r1) {
         uint4 ws[T];
 #pragma unroll
         for (int t = 0; t < T; ++t) ws[t] = *reinterpret_cast<const uint4*>(L.wsg + 512 * t + 8 * lane);
-        for (int r = rb + static_cast<int>(blockIdx.x); r < r1; r += gridDim.x) {
+        for (int r = rb + job; r < r1; r += jobs) {
             uint4 xs[T];
             load_row(r, xs);
             float a = 0.0f;
@@ -100,14 +105,15 @@ __global__ __launch_bounds__(64 * kLogitsWaves) void k_logits_rows(LayerDev L, M
             if (lane == 0) B.sgate[r] = rbf(1.0f / (1.0f + expf(-rbf(a))));
         }
     }
-    for (int r = rb + wave; r < r1; r += kLogitsWaves) {
+    int mine = rb + job;  // the next row whose copies this wave writes
+    for (int r = rb; r < r1; ++r) {
         uint4 xv[T];
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             xv[t] = xa[t];
             xa[t] = xb[t];
         }
-        load_row(r + 2 * kLogitsWaves < r1 ? r + 2 * kLogitsWaves : r1 - 1, xb);
+        load_row(r + 2 < r1 ? r + 2 : r1 - 1, xb);
         float acc[NE];
 #pragma unroll
         for (int n = 0; n < NE; ++n) acc[n] = 0.0f;
@@ -135,7 +141,8 @@ __global__ __launch_bounds__(64 * kLogitsWaves) void k_logits_rows(LayerDev L, M
                 B.logits[static_cast<size_t>(r) * L.E + e] = L.rbias ? lg + rbias[s] : lg;
             }
         }
-        if (store_x) {
+        if (store_x && r == mine) {
+            mine += jobs;
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 const size_t at = static_cast<size_t>(r) * H + 512 * t + 8 * lane;
@@ -1238,11 +1245,10 @@ hipError_t launch_router_rows_t(const LayerDev& L, const MoeBufs& B, int M, cons
         slots = nb * router_cus();
         resident.store(slots, std::memory_order_relaxed);
     }
-    // request rows per workgroup: the grid fills the resident slots once (at least one row
-    // per wave)
-    const int gx = (L.E + NE - 1) / NE;
+    // request rows per workgroup: the grid fills the resident slots once
+    const int gx = (L.E + NE * kLogitsWaves - 1) / (NE * kLogitsWaves);
     int gy = slots / gx;
-    gy = gy < 1 ? 1 : gy > (M + kLogitsWaves - 1) / kLogitsWaves ? (M + kLogitsWaves - 1) / kLogitsWaves : gy;
+    gy = gy < 1 ? 1 : gy > M ? M : gy;
     const int rpw = (M + gy - 1) / gy;
     gy = (M + rpw - 1) / rpw;
     const int planar = prefill_planes(L, M) == 2 ? 1 : 0;

@@ -195,6 +195,24 @@ def test_prefill_512_zipf_group64(gpu, q38, orc):
         L.close()
 
 
+@pytest.mark.parametrize("H,E,M", [(512, 64, 17), (1536, 192, 40), (2048, 448, 19), (4096, 64, 33)])
+def test_prefill_router_shapes(gpu, q38, orc, H, E, M):
+    """Router logits bit for bit where the last workgroup's waves have no router rows left (8, 4
+    or 2 per wave), rows fill the grid once, twice or in part, and every row's copies and shared
+    gate are written by some wave (the outputs)."""
+    geo = dict(hidden=H, inter=512, experts=E, top_k=4)
+    L = q38.MoeLayer(gpu, q38.desc(**geo), seed=SEED, layer=LAYER)
+    try:
+        x = orc.rmsnorm(orc.embed(SEED, tokens(M), H))
+        y, ex, wt, lg, plan = run_forward(q38, L, q38.desc(**geo), x)
+        wy, wex, wwt, wlg = orc.moe_layer_synth(oracle_lib.make_desc(**geo), SEED, LAYER, x)
+        assert np.array_equal(lg.view(np.uint32), wlg.view(np.uint32))
+        assert np.array_equal(ex, wex) and np.array_equal(wt.view(np.uint32), wwt.view(np.uint32))
+        tol_check(orc, y, wy)
+    finally:
+        L.close()
+
+
 @pytest.mark.parametrize("groups", [(64, 64), (64, None), (None, 64)])
 @pytest.mark.parametrize("M", [17, 33])
 def test_prefill_group64_segments(gpu, q38, orc, groups, M):
