@@ -202,8 +202,9 @@ void q38_set_fused_layers(int enable);
  * verify-width decode, src/vq_metal_kernels.hpp:564-579, which forms w = q * scale (+ bias)
  * per weight): one 8-byte entry per subvector from a book held whole in LDS, the
  * per-dimension scale applied to the inputs and the bias as a per-row sum. 0: none (the
- * decoded fp16 book on the other kernels); 1 (default): 5-16 rows, and 1-4 rows where the
- * one-launch layer kernel is not taken (it is faster at those widths); 2: 1-16 rows.
+ * decoded fp16 book on the other kernels); 1 (default): the widths at which they are the faster
+ * ones (1-4 rows where the one-launch layer kernel is not taken, 5-16 rows where the segmented
+ * kernels are not: other than 512 experts); 2: 1-16 rows.
  * No counterpart in the reference. */
 void q38_set_u8_native(int mode);
 

@@ -504,8 +504,8 @@ static void fill_dev_mixed(q38_moe_layer* L, const q38_moe_mixed_weights* w) {
         v.pb[p][1] = b;
         v.p[p] = b;
     }
-    // the odd bank (two codebook chunks) writes two partial-sum planes, the even bank writes
-    // one and clears the second
+    // both banks write two partial-sum planes, one per chunk (the d4 bank's: the even and the odd
+    // subvectors)
     v.gu_parts = v.d_parts = 2;
 }
 

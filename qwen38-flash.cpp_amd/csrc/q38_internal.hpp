@@ -140,7 +140,8 @@ struct LayerDev {
     // H 2048, I 512, per-row scales, no affine shared expert). call_path: the kernels of this
     // verify call (moe_call_dev). kPathU8: those (1-16 rows while they are enabled), one
     // partial-sum plane; kPathSeg: the segmented LDS-codebook kernels of the prefill widths (5-16
-    // rows; mixed layers at any), two planes, the router storing the fp16 rows chunk-planar; kPathOther: the others.
+    // rows; mixed layers at any), two planes, the router storing the fp16 rows chunk-planar;
+    // kPathOther: the others.
     int u8_native, call_path;
 };
 enum { kPathOther = 0, kPathU8 = 1, kPathSeg = 2 };
@@ -291,8 +292,8 @@ bool moe_uses_seg_verify(const LayerDev& L, int M);
 LayerDev moe_call_dev(const LayerDev& L, int M);
 // Verify widths (1-16 rows) of layers with U8 books on the kernels that read the books
 // themselves (k_gu_u8, k_swiglu_u8, k_dn_u8), by mode: 0 never (the decoded fp16 books on the
-// other verify kernels), 1 (default) at 5-16 rows and at 1-4 rows where the one-launch layer
-// is not taken, 2 at every verify width.
+// other verify kernels), 1 (default) where they are faster: at 5-16 rows where the segmented kernels
+// are not taken, at 1-4 rows where the one-launch layer is not; 2 at every verify width.
 bool moe_u8_call(const LayerDev& L, int M);
 void set_u8_native(int mode);
 // The U8 kernels' operands of a per-dimension book: u = q (+ 128 when centred) as bytes and

@@ -14,9 +14,9 @@
 //   k_down_mfma   SwiGLU of the gate/up sums + down projection (R7, R8), same scheme.
 //   k_combine     ordered route reduction (slot order) + shared expert x sigmoid gate +
 //                 merge (R8, R10, R11); in a chain it adds the residual in place.
-// Rows <= 4 take the narrow kernels of q38_moe4.hip instead of k_topk_plan + k_*_mfma.
-// Mixed layers (two codebook geometries by expert parity) run k_gu_mfma / k_down_mfma once
-// per bank. Layers with per-64-input scale groups use the k_*_grouped VALU kernels.
+// Rows <= 4 take the narrow kernels of q38_moe4.hip instead of k_topk_plan + k_*_mfma; 5-16 rows of
+// d8/14-bit layers with 512 experts, and mixed layers, the segmented kernels of q38_moe_pf.hip.
+// Other layers with scale groups, d4 and d2 codes use the k_*_grouped VALU kernels.
 #ifdef Q38_TRACE
 #define g_trace g_trace_route  // (each code object holds its own stamp buffer)
 #endif
@@ -494,7 +494,6 @@ __device__ __forceinline__ const uint4* xs_lane(const uint4* xs, int xrow, int z
     return reinterpret_cast<const uint4*>(reinterpret_cast<const unsigned char*>(xs) +
                                           (active ? xrow : zero_row) * XsLayout<NSUB>::RB + q * XsLayout<NSUB>::QB);
 }
-
 
 template <int BITS, int NSUB, int NCHUNK>
 __global__ __launch_bounds__(kMfmaThreads) void k_gu_mfma(LayerDev L, MoeBufs B, int M) {
@@ -1258,8 +1257,11 @@ bool moe_u8_call(const LayerDev& L, int M) {
     if (!L.u8_native || L.shared_affine || L.mixed || M < 1 || M > kMaxRows) return false;
     const int mode = g_u8_native.load(std::memory_order_relaxed);
     if (mode == 0) return false;
-    if (mode == 2 || M > 4) return true;
-    // 1-4 rows: the one-launch layer on the decoded book is faster wherever it is taken
+    if (mode == 2) return true;
+    // 5-16 rows: the segmented kernels on the decoded book are faster wherever they are taken (per
+    // layer, U8 kernels against them: 5 rows 54 and 38 us, 9 rows 79 and 51, 16 rows 119 and 72);
+    // 1-4 rows: the one-launch layer on it
+    if (M > 4) return !moe_uses_seg_verify(L, M);
     LayerDev d = L;
     d.fused_mode = 0;
     return !moe_uses_fused(d, M);
@@ -1273,8 +1275,6 @@ hipError_t launch_u8_operands(const void* q, int K, int centered, const uint16_t
     return hipGetLastError();
 }
 
-// Mixed layers run their two banks on the MFMA kernels: H = 2048, I = 512, per-row scales,
-// chunked fp16 codebooks prepared for both banks.
 bool moe_plans_in_gate_up(const LayerDev& L, int M) {
     if (L.call_path == kPathSeg) return false;
     return moe_uses_mfma(L) || moe_uses_narrow(L, M);

@@ -6,7 +6,7 @@ widths (1, 4, 16 rows), prefill width and with per-64-input scale groups.
 At 1-16 rows such layers run on the kernels that read the U8 books themselves (the reference's
 verify-width decode, src/vq_metal_kernels.hpp:564-579): checked against the oracle's float
 decode and against the decoded-fp16-book kernels (q38_set_u8_native(0)) on the same rows
-(mode 2 takes them at 1-4 rows too; the default takes them at 5-16)."""
+(mode 2; the default takes them where neither the one-launch layer nor the segmented kernels run)."""
 import ctypes as C
 
 import numpy as np
@@ -95,6 +95,21 @@ def test_u8_kernels_vs_decoded_book(u8layer, q38, orc, restore_u8_native, M):
     r0 = tol_check(orc, y0, wy)
     print(f"M={M}: U8 kernels rel {r1[0]:.2e} max {r1[1]:.2e}; decoded book rel {r0[0]:.2e} max {r0[1]:.2e}")
     assert not np.array_equal(y1, y0)
+
+
+@pytest.mark.parametrize("M", [5, 8, 9, 16])
+def test_default_mode_takes_the_segmented_kernels(u8layer, q38, orc, restore_u8_native, M):
+    """5-16 rows in the default mode: the bits of the decoded-book kernels, within the MoE
+    tolerance of the oracle's float decode."""
+    x = orc.rmsnorm(orc.embed(SEED, [300 + 5 * i for i in range(M)], 2048))
+    q38.lib.q38_set_u8_native(0)
+    y0 = run_forward(q38, u8layer, u8layer.desc, x)[0]
+    q38.lib.q38_set_u8_native(1)
+    y1, ex1, wt1, lg1, plan1 = run_forward(q38, u8layer, u8layer.desc, x)
+    wy, wex, wwt, wlg = orc.moe_layer_synth(oracle_lib.make_desc(book_format=2), SEED, 9, x)
+    assert np.array_equal(ex1, wex) and np.array_equal(wt1, wwt)
+    assert np.array_equal(y1, y0)
+    tol_check(orc, y1, wy)
 
 
 def test_u8_kernels_repeat_and_width_change(u8layer, q38, orc, restore_u8_native):
