@@ -509,37 +509,25 @@ static void fill_dev_mixed(q38_moe_layer* L, const q38_moe_mixed_weights* w) {
     v.gu_parts = v.d_parts = 2;
 }
 
-// A mixed layer's operands of the segmented kernels: chunked fp16 codebooks (the d4 books are
-// already in the chunk layout, [1][256][4]; the INT8 d8 books are decoded, q * scale, into
-// [2][16384][4] fp16) and both banks' codes in the tiled layout those kernels load from (one more
-// copy of the codes, as for the uniform layers).
+// Chunked fp16 codebooks of a mixed layer for the segmented kernels, which copy them into LDS 16
+// bytes at a time: the INT8 d8 books decoded (q * scale) into [2][16384][4] fp16, the d4 books,
+// already in the chunk layout ([1][256][4]), copied to an aligned place. The codes stay where the
+// caller holds them.
 static int prepare_mixed(q38_moe_layer* L) {
-    const size_t per = align256(static_cast<size_t>(16384) * 8 * 2);
-    LayerDev& v = L->dev;
-    size_t total = 3 * per, off[3][2];
-    int64_t rows[3][2];
-    for (int p = 0; p < 3; ++p)
-        for (int b = 0; b < 2; ++b) {
-            // bank 0: the even experts and the shared one (E); bank 1: the odd experts
-            const int experts = L->desc.experts / 2 + (b == 0 && L->desc.has_shared ? 1 : 0);
-            rows[p][b] = static_cast<int64_t>(experts) * (p < 2 ? L->desc.inter : L->desc.hidden);
-            off[p][b] = total;
-            total += align256(static_cast<size_t>(rows[p][b]) * v.pb[p][b].words * 4);
-        }
+    const size_t per = align256(static_cast<size_t>(16384) * 8 * 2), small = align256(256 * 4 * 2);
     char* base = nullptr;
-    if (hipMalloc(&base, total) != hipSuccess) return fail(Q38_ENOMEM, "hipMalloc failed for prepared codebooks");
+    if (hipMalloc(&base, 3 * (per + small)) != hipSuccess)
+        return fail(Q38_ENOMEM, "hipMalloc failed for prepared codebooks");
     hipError_t e = hipSuccess;
+    LayerDev& v = L->dev;
     for (int p = 0; p < 3 && e == hipSuccess; ++p) {
-        auto* dst = reinterpret_cast<uint16_t*>(base + p * per);
+        auto* dst = reinterpret_cast<uint16_t*>(base + p * (per + small));
+        auto* dst4 = reinterpret_cast<uint16_t*>(base + p * (per + small) + per);
         e = launch_split_book_i8(v.pb[p][1].book_i8, v.pb[p][1].book_scale, 1 << v.pb[p][1].bits, v.pb[p][1].dim, dst,
                                  nullptr);
-        v.pb[p][0].book4 = v.pb[p][0].book;
+        if (e == hipSuccess) e = hipMemcpyAsync(dst4, v.pb[p][0].book, 256 * 4 * 2, hipMemcpyDeviceToDevice, nullptr);
+        v.pb[p][0].book4 = dst4;
         v.pb[p][1].book4 = dst;
-        for (int b = 0; b < 2 && e == hipSuccess; ++b) {
-            auto* ct = reinterpret_cast<uint32_t*>(base + off[p][b]);
-            e = launch_tile_codes(v.pb[p][b].codes, rows[p][b], v.pb[p][b].words, v.pb[p][b].bits, ct, nullptr);
-            v.pb[p][b].codes_t = ct;
-        }
         v.p[p] = v.pb[p][1];
     }
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);

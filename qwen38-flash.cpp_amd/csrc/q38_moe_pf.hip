@@ -642,17 +642,12 @@ __device__ __forceinline__ uint32_t code14_x8(const uint32_t* w, int q) {
 
 // d4/8-bit codes (the even bank of mixed layers): subvectors 2 t and 2 t + 1 of four dims are the
 // chunks of an 8-dim subvector t, so chunk c of the layer takes every second byte and the inputs
-// keep the chunk-planar layout. A lane's span of SPL subvectors t is 2 SPL / 32 blocks of 8 words;
-// each word, shifted by 8 c, holds the codes of a pair of t in bytes 0 and 2.
-template <int SPL>
-__device__ __forceinline__ void seg_load_bytes(const uint32_t* codes_t, int blocks, size_t tile64, int rr, int span,
-                                               uint32_t (&w)[SPL / 2]) {
-    const uint32_t* base = codes_t + (tile64 * blocks + span * (SPL / 16)) * (8 * 64) + rr * 4;
-#pragma unroll
-    for (int c = 0; c < SPL / 8; ++c) {  // (two chunks of 4 words per block)
-        const uint4 v = *reinterpret_cast<const uint4*>(base + c * 256);
-        w[4 * c] = v.x; w[4 * c + 1] = v.y; w[4 * c + 2] = v.z; w[4 * c + 3] = v.w;
-    }
+// keep the chunk-planar layout; each word, shifted by 8 c, holds the codes of a pair of t in bytes
+// 0 and 2. Mixed layers hold no tiled copy of their codes: a lane loads its span's NW words from
+// the caller's rows (4-byte aligned).
+template <int NW>
+__device__ __forceinline__ void seg_load_row(const uint32_t* p, uint32_t (&w)[NW]) {
+    __builtin_memcpy(w, p, NW * 4);
 }
 
 // The LDS byte offsets of the entries of subvectors 2 t, 2 t + 1.
@@ -884,9 +879,11 @@ __device__ __forceinline__ void gu_seg_body(const LayerDev& L, const MoeBufs& B,
         const size_t row0 = static_cast<size_t>(expert) * I + tile * TR + rg * 32;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int rr = static_cast<int>(row0 & 63) + 16 * i + r16;
-            if constexpr (BITS == 14) seg_load_codes<32>(P.codes_t, KS, row0 >> 6, rr, kh * 4 + q, 0, w[i]);
-            else seg_load_bytes<32>(P.codes_t, 2 * KS, row0 >> 6, rr, kh * 4 + q, w[i]);
+            if constexpr (PAR >= 0)
+                seg_load_row(P.codes + (row0 + 16 * i + r16) * (4 * KP * NW) + (kh * 4 + q) * NW, w[i]);
+            else
+                seg_load_codes<32>(P.codes_t, KS, row0 >> 6, static_cast<int>(row0 & 63) + 16 * i + r16, kh * 4 + q, 0,
+                                   w[i]);
         }
     };
     if constexpr (G8) {
@@ -1023,9 +1020,10 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
     gu_seg_body<NSUB, G8, 14, -1>(L, B, M, L.p[proj], proj, chunk, (gridDim.x / 32) * 8, (kk >> 2) * 8 + x8, S);
 }
 // Both banks of a mixed layer in one launch: workgroup types bank x projection x chunk, half of
-// the workgroups each bank (an item costs its gathers, the same number in both). 16 rows: 32 us,
-// and 19 us for the down kernel, against 41 + 26 and 28 + 24 us of 16-row kernels that ran one
-// bank after the other, staged their operand rows and, for the d4 bank, cleared the second plane.
+// the workgroups each bank (an item costs its gathers, the same number in both). 16 rows: 35 us,
+// and 21 us for the down kernel, against 41 + 26 and 28 + 24 us of 16-row kernels that ran one
+// bank after the other, staged their operand rows and, for the d4 bank, cleared the second plane
+// (32 and 19 us from a tiled copy of the codes, which would double the layer's memory).
 __global__ __launch_bounds__(kSegThreads) void k_gu_seg_mixed(LayerDev L, MoeBufs B, int M) {
     __shared__ GuSegLds<256> S;
     touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
@@ -1096,9 +1094,11 @@ __device__ __forceinline__ void dn_seg_body(const LayerDev& L, const MoeBufs& B,
         const size_t row0 = static_cast<size_t>(expert) * H + tile * TR + rg * 32;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int rr = static_cast<int>(row0 & 63) + 16 * i + r16;
-            if constexpr (BITS == 14) seg_load_codes<SPL>(P.codes_t, KS, row0 >> 6, rr, blk, half, w[i]);
-            else seg_load_bytes<SPL>(P.codes_t, 2 * KS, row0 >> 6, rr, q, w[i]);
+            if constexpr (PAR >= 0)
+                seg_load_row(P.codes + (row0 + 16 * i + r16) * (4 * NW) + q * NW, w[i]);
+            else
+                seg_load_codes<SPL>(P.codes_t, KS, row0 >> 6, static_cast<int>(row0 & 63) + 16 * i + r16, blk, half,
+                                    w[i]);
         }
     };
     if constexpr (G8) {
@@ -1331,13 +1331,12 @@ int prefill_planes(const LayerDev& L, int M) {
     return 2;
 }
 
-// Mixed layers (verify widths; H 2048, I 512, row scales): both banks' codes tiled and books in
-// chunks.
+// Mixed layers (verify widths; H 2048, I 512, row scales): both banks' books in chunks.
 static bool moe_mixed_seg(const LayerDev& L) {
     if (!L.mixed || L.H != 2048 || L.I != 512) return false;
     for (int p = 0; p < 3; ++p)
         for (int b = 0; b < 2; ++b)
-            if (L.pb[p][b].ngrp != 1 || !L.pb[p][b].book4 || !L.pb[p][b].codes_t) return false;
+            if (L.pb[p][b].ngrp != 1 || !L.pb[p][b].book4) return false;
     return true;
 }
 

@@ -152,3 +152,52 @@ def test_explicit_mixed_layer_equals_synthetic(gpu, q38, mixed_stack, M):
         assert q38.lib.q38_moe_layer_create_mixed(gpu.h, C.byref(d), C.byref(w), C.byref(h2)) == q38.Q38_EINVAL
     finally:
         q38.lib.q38_moe_layer_destroy(h)
+
+
+def mixed_layer(q38, gpu, w):
+    h = C.c_void_p()
+    d = mixed_desc(q38)
+    q38.check(q38.lib.q38_moe_layer_create_mixed(gpu.h, C.byref(d), C.byref(w), C.byref(h)))
+    return h
+
+
+def test_creation_keeps_the_codes_where_they_are(gpu, q38, mixed_stack):
+    """A mixed layer holds its chunked codebooks (3 x 256 KiB) and no second copy of the packed
+    codes (about 378 MB)."""
+    import torch
+    w = q38.MoeMixedWeights()
+    q38.check(q38.lib.q38_moe_layer_mixed_weights(mixed_stack[0].h, C.byref(w)))
+    q38.lib.q38_moe_layer_destroy(mixed_layer(q38, gpu, w))  # (what a first creation loads)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    h = mixed_layer(q38, gpu, w)
+    try:
+        assert before - torch.cuda.mem_get_info()[0] <= 16 << 20
+    finally:
+        q38.lib.q38_moe_layer_destroy(h)
+
+
+def test_tensors_on_element_addresses(gpu, q38, mixed_stack):
+    """Packed codes and d4 books on 4-byte addresses give the bits of the aligned tensors."""
+    src = mixed_stack[7]
+    w = q38.MoeMixedWeights()
+    q38.check(q38.lib.q38_moe_layer_mixed_weights(src.h, C.byref(w)))
+    keep = []
+
+    def shifted(ptr, words):
+        t = G.to_dev(np.concatenate([np.zeros(1, np.uint32), G.d2h(ptr, words, np.uint32)]))
+        keep.append(t)
+        return t.data_ptr() + 4
+
+    for p, (rows, n) in enumerate(((512, 2048), (512, 2048), (2048, 512))):
+        w.codes_d4[p] = shifted(w.codes_d4[p], 257 * rows * (n // 4 // 32) * 8)
+        w.codes_d8[p] = shifted(w.codes_d8[p], 256 * rows * (n // 8 // 32) * 14)
+        w.books_d4[p] = shifted(w.books_d4[p], 512)
+    L = type("Explicit", (), dict(h=mixed_layer(q38, gpu, w)))()
+    try:
+        x = np.random.default_rng(9).normal(0, 1, (5, 2048)).astype(np.float32)
+        xb = (x.view(np.uint32) >> 16).astype(np.uint16)
+        for u, v in zip(run_forward(q38, src, mixed_desc(q38), xb), run_forward(q38, L, mixed_desc(q38), xb)):
+            assert np.array_equal(u, v)
+    finally:
+        q38.lib.q38_moe_layer_destroy(L.h)
