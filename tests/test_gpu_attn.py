@@ -203,6 +203,29 @@ def test_one_hot_query_reads_its_key_exactly(gpu, q38, orc):
     assert np.array_equal(out, wout)
 
 
+@pytest.mark.parametrize("T0", [12, 4099])
+def test_subnormal_probabilities(gpu, q38, orc, T0):
+    """A probability below the smallest normal number (exp(-88) = 6.05e-39, 66 steps of 2^-133 in
+    bf16) still weighs its value: 2^126 in one token, 0 in all others. Tolerance: one such step
+    (2^-133 x 2^126 = 2^-7) and the two bf16 roundings after it."""
+    j = 40
+    L = identity_layer(q_rows={j: (0, 3), 2 * D_ID + j: (0, 3)})  # (both heads)
+    keys, values = L.random_cache(np.random.default_rng(3), T0 + 4, T0)
+    keys[:, :T0] = values[:, :T0] = 0
+    keys[0, 5, j] = to16(np.array([88.0]), 0)[0]
+    values[0, T0 - 1, :] = to16(np.full(D_ID, 2.0 ** 126), 0)
+    x = np.zeros((1, H_ID), np.uint16)
+    x[0, 0] = to16(np.array([1.0]), 0)[0]
+    dev = DevAttn(q38, gpu, L, T0 + 4)
+    try:
+        got = bf(dev.verify(x, dev.cache_dev(keys, values), T0, 3)[0])
+    finally:
+        dev.close()
+    want = bf(orc.attn_verify(L, x, keys, values, T0, 3)[0][0])
+    assert (want > 0.25).all()
+    assert (np.abs(got - want) <= 2.0 ** -7 + want * 2.0 ** -7).all(), (got, want)
+
+
 def test_limits_and_geometry(gpu, q38):
     L = AttnLayer(seed=6)
     dev = DevAttn(q38, gpu, L, 32)
