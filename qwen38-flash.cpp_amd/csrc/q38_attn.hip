@@ -52,10 +52,10 @@ constexpr int64_t kSliceWgs = 256;
 __device__ __forceinline__ float tbf(float v) { return bf2f(f2bf(v)); }
 __device__ __forceinline__ float sigmoid_bf(float x) { return tbf(1.0f / (1.0f + expf(-x))); }
 
-// Two floats rounded to bf16 (nearest even), packed lo first, in one instruction.
+// Two floats rounded to bf16 (nearest even, as rbf_cvt), packed lo first, in one instruction.
 __device__ __forceinline__ uint32_t pack_bf(float lo, float hi) {
     typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
-    const bf2_t v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
+    const bf2_t v = {static_cast<__bf16>(own(lo)), static_cast<__bf16>(own(hi))};
     return __builtin_bit_cast(uint32_t, v);
 }
 // exp(x) for x <= 0 within one unit in the last place, subnormal results included: 2^(k + f) for

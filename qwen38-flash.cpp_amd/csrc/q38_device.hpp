@@ -55,8 +55,15 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
     return static_cast<uint16_t>((x & 0x7fffffffu) > 0x7f800000u ? quiet : rounded);
 }
 __device__ __forceinline__ float rbf(float f) { return bf2f(f2bf(f)); }
-// rbf by the conversion instruction (the same nearest-even rounding, two instructions).
-__device__ __forceinline__ float rbf_cvt(float f) { return static_cast<float>(static_cast<__bf16>(f)); }
+// rbf by the conversion instruction: the same nearest-even rounding (equal to the integer form on
+// all 2^32 patterns), two instructions. `own` hides how f was formed: under floating-point
+// contraction the compiler folds double -> float -> bf16 into one rounding of the double, and the
+// results then differ from the two roundings of the contract where the first one makes a tie.
+__device__ __forceinline__ float own(float f) {
+    asm("" : "+v"(f));
+    return f;
+}
+__device__ __forceinline__ float rbf_cvt(float f) { return static_cast<float>(static_cast<__bf16>(own(f))); }
 __device__ __forceinline__ float h2f(uint16_t h) { return static_cast<float>(__builtin_bit_cast(_Float16, h)); }
 __device__ __forceinline__ uint16_t f2h(float f) { return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f)); }
 
