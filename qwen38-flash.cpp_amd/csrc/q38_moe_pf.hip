@@ -498,8 +498,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // a 16-byte cache line read. Work units are (expert slot, pass of up to 16 of the slot's
 // routes); items are (unit, tile of output rows), and each workgroup walks a contiguous
 // range of items, so the B operand (the pass's 16 route rows, this chunk's dims) stays in
-// registers for all tiles of a unit. Wave (kh, rg): K part kh (lane quarter q owns one 16-
-// or 32-code span of each of its rows) x row group rg (32 rows = two 16-row MFMA tiles);
+// registers for all tiles of a unit. Wave (kh, rg): K part kh (lane quarter q owns one span of
+// codes of each of its rows, 32 in gate/up, 16 in down) x row group rg (32 rows = two 16-row MFMA tiles);
 // v_mfma_f32_16x16x32_f16 with A = the two gathered 4-dim entries of subvectors 2t, 2t + 1
 // of the lane's span and B = the same subvectors' dims of route c16, read as one 16-byte
 // word from the chunk-planar fp16 inputs. K parts are summed through LDS in part order.
@@ -759,7 +759,7 @@ __device__ __forceinline__ void seg_mfma_g8(const uint32_t (&pr)[2][8], const ui
     for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(acc[i]));
 }
 
-// The products of one item (NSUB-independent): codes w of its two 16-row tiles (SPL 32: the
+// The products of one item: codes w of its two 16-row tiles (SPL 32: the
 // lane's 14 words, SPL 16: its 7), the next item's words loaded into w by next(half) as soon as
 // a half has become pairs.
 template <int SPL, int NG, typename F>
@@ -812,28 +812,26 @@ __device__ __forceinline__ void seg_range(int n_items, int per_type, int idx, in
     i1 = static_cast<int>(static_cast<int64_t>(idx + 1) * n_items / per_type);
 }
 
-// Gate/up (NSUB = H / 8 subvectors per row: 128 or 256; at 512 the K-part partial sums of
-// four K parts would not fit in LDS beside the 128 KiB codebook chunk). Output rows of an item:
-// TR = 32 * RG rows of I; chunk `chunk` of projection `proj` per workgroup type. B = rows of
+// Gate/up (H 2048: 256 subvectors per row, two K parts of 128). Output rows of an item: TR =
+// 32 * RG = 128 rows of I; chunk `chunk` of projection `proj` per workgroup type. B = rows of
 // the chunk-planar fp16 inputs ([2][M][H / 2]).
 // G8: one scale per 64 inputs (ngrp = H / 64) instead of one per output row. PAR >= 0: the bank of
 // a mixed layer (BITS 8: the even one).
-template <int NSUB>
+constexpr int kGuParts = 2, kGuGroups = 4, kGuTile = 32 * kGuGroups;  // (eight waves)
 struct GuSegLds {
-    static constexpr int KP = NSUB / 128, RG = 8 / KP, RED = 2 * (KP - 1) * RG * 2 * 64;
+    static constexpr int RED = 2 * (kGuParts - 1) * kGuGroups * 2 * 64;
     // One static LDS block (the codebook chunk at offset 0, known when compiling, so a gather's
     // address is its code offset alone), the K-part partial sums ([2][KP - 1][RG][2][64]) and
     // the unit table.
     uint2 book[kSegKent];
-    f4_t red[RED > 0 ? RED : 1];
+    f4_t red[RED];
     SegTab T;
 };
-template <int NSUB, bool G8, int BITS, int PAR>
+template <bool G8, int BITS, int PAR>
 __device__ __forceinline__ void gu_seg_body(const LayerDev& L, const MoeBufs& B, int M, const ProjDev& P, int proj,
-                                            int chunk, int per_type, int idx, GuSegLds<NSUB>& S) {
-    constexpr int KP = NSUB / 128, RG = 8 / KP, TR = 32 * RG, KS = NSUB / 32, KENT = 1 << BITS;
+                                            int chunk, int per_type, int idx, GuSegLds& S) {
+    constexpr int KP = kGuParts, RG = kGuGroups, TR = kGuTile, KS = 8, KENT = 1 << BITS;
     constexpr int NW = BITS == 14 ? 14 : 16;  // words of a lane's 32-subvector span
-    static_assert(NSUB % 128 == 0 && KP * RG == 8, "8 waves = K parts x row groups");
     unsigned char* lds = reinterpret_cast<unsigned char*>(S.book);
     const unsigned char* book = lds;
     f4_t* red = S.red;
@@ -891,7 +889,7 @@ __device__ __forceinline__ void gu_seg_body(const LayerDev& L, const MoeBufs& B,
 #pragma unroll
             for (int i = 0; i < 2; ++i)
                 seg_load_scales<16>(P.scales + (static_cast<size_t>(expert) * I + tile * TR + rg * 32 + 16 * i + r16) *
-                                                   (NSUB / 8) + kh * 16, sc[i]);
+                                                   (16 * KP) + kh * 16, sc[i]);
         };
         uint4 bx[16];
         uint32_t w[2][14], sn[2][8];
@@ -923,12 +921,10 @@ __device__ __forceinline__ void gu_seg_body(const LayerDev& L, const MoeBufs& B,
             }, acc);
             if (new_unit) load_b(k + 1, bx);
             const int buf = item & 1;
-            if (KP > 1) {
-                if (kh > 0)
+            if (kh > 0)
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) red[(((buf * (KP - 1) + kh - 1) * RG + rg) * 2 + i) * 64 + lane] = acc[i];
-                lds_barrier();
-            }
+                for (int i = 0; i < 2; ++i) red[(((buf * (KP - 1) + kh - 1) * RG + rg) * 2 + i) * 64 + lane] = acc[i];
+            lds_barrier();
             if (kh == 0)
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
@@ -977,12 +973,10 @@ __device__ __forceinline__ void gu_seg_body(const LayerDev& L, const MoeBufs& B,
         // second register set would not fit), in flight through the reduction and stores
         if (new_unit) load_b(k + 1, bx);
         const int buf = item & 1;
-        if (KP > 1) {
-            if (kh > 0)
+        if (kh > 0)
 #pragma unroll
-                for (int i = 0; i < 2; ++i) red[(((buf * (KP - 1) + kh - 1) * RG + rg) * 2 + i) * 64 + lane] = acc[i];
-            lds_barrier();  // (the other buffer was read before the previous item's barrier)
-        }
+            for (int i = 0; i < 2; ++i) red[(((buf * (KP - 1) + kh - 1) * RG + rg) * 2 + i) * 64 + lane] = acc[i];
+        lds_barrier();  // (the other buffer was read before the previous item's barrier)
         if (kh == 0) {
             const int j = un.w + r16;
 #pragma unroll
@@ -1010,14 +1004,14 @@ __device__ __forceinline__ void gu_seg_body(const LayerDev& L, const MoeBufs& B,
     }
 }
 
-template <int NSUB, bool G8>
+template <bool G8>
 __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, int M) {
-    __shared__ GuSegLds<NSUB> S;
+    __shared__ GuSegLds S;
     touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
     const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
     const int type = kk & 3, proj = type >> 1, chunk = type & 1;
     // (the chunk-0 and chunk-1 workgroups of an index share an XCD)
-    gu_seg_body<NSUB, G8, 14, -1>(L, B, M, L.p[proj], proj, chunk, (gridDim.x / 32) * 8, (kk >> 2) * 8 + x8, S);
+    gu_seg_body<G8, 14, -1>(L, B, M, L.p[proj], proj, chunk, (gridDim.x / 32) * 8, (kk >> 2) * 8 + x8, S);
 }
 // Both banks of a mixed layer in one launch: workgroup types bank x projection x chunk, half of
 // the workgroups each bank (an item costs its gathers, the same number in both). 16 rows: 35 us,
@@ -1025,29 +1019,28 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
 // bank after the other, staged their operand rows and, for the d4 bank, cleared the second plane
 // (32 and 19 us from a tiled copy of the codes, which would double the layer's memory).
 __global__ __launch_bounds__(kSegThreads) void k_gu_seg_mixed(LayerDev L, MoeBufs B, int M) {
-    __shared__ GuSegLds<256> S;
+    __shared__ GuSegLds S;
     touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
     const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
     const int type = kk & 7, proj = (type >> 1) & 1, chunk = type & 1;
     const int per_type = (gridDim.x / 64) * 8, idx = (kk >> 3) * 8 + x8;
-    if (type & 4) gu_seg_body<256, false, 14, 1>(L, B, M, L.pb[proj][1], proj, chunk, per_type, idx, S);
-    else gu_seg_body<256, false, 8, 0>(L, B, M, L.pb[proj][0], proj, chunk, per_type, idx, S);
+    if (type & 4) gu_seg_body<false, 14, 1>(L, B, M, L.pb[proj][1], proj, chunk, per_type, idx, S);
+    else gu_seg_body<false, 8, 0>(L, B, M, L.pb[proj][0], proj, chunk, per_type, idx, S);
 }
 
-// Down (NSUB = I / 8 subvectors per row: 64 or 128; SPL = NSUB / 4 per lane quarter, 16 =
-// half a code block). One K part: wave rg owns rows 32 rg .. + 31 of a TR = 256-row tile of
-// H. B = the pass's SwiGLU rows (chunk-planar fp16 at sorted positions); outputs at the
+// Down (I 512: 64 subvectors per row, SPL = 16 per lane quarter, half a code block). One K part:
+// wave rg owns rows 32 rg .. + 31 of a TR = 256-row tile of H. B = the pass's SwiGLU rows (chunk-planar fp16 at sorted positions); outputs at the
 // route index.
+constexpr int kDnTile = 256;
 struct DnSegLds {  // one static LDS block, as for gate/up
     uint2 book[kSegKent];
     SegTab T;
 };
-template <int NSUB, bool G8, int BITS, int PAR>
+template <bool G8, int BITS, int PAR>
 __device__ __forceinline__ void dn_seg_body(const LayerDev& L, const MoeBufs& B, int M, const ProjDev& P, int chunk,
                                             int per_type, int idx, DnSegLds& S) {
-    constexpr int SPL = NSUB / 4, TR = 256, KS = NSUB / 32, KENT = 1 << BITS;
-    static_assert(SPL == 16 || SPL == 32, "16-code or 32-code lane spans");
-    constexpr int NB = SPL / 2, NW = BITS == 8 ? SPL / 2 : SPL == 32 ? 14 : 7;
+    constexpr int SPL = 16, TR = kDnTile, KS = 2, KENT = 1 << BITS;
+    constexpr int NB = SPL / 2, NW = BITS == 8 ? 8 : 7;
     unsigned char* lds = reinterpret_cast<unsigned char*>(S.book);
     const unsigned char* book = lds;
     SegTab& T = S.T;
@@ -1073,7 +1066,7 @@ __device__ __forceinline__ void dn_seg_body(const LayerDev& L, const MoeBufs& B,
     float* dout = B.d + chunk * B.d_plane;
     const int MKM = M * K + (hs ? M : 0);
     const uint16_t* hplane = B.h16 + static_cast<size_t>(chunk) * MKM * (I / 2);
-    const int blk = SPL * q / 32, half = SPL == 16 ? (q & 1) : 0;
+    const int blk = q >> 1, half = q & 1;
 
     // SwiGLU operand of unit k: row (sorted position) of route j0 + r16, subvectors SPL q +
     // (0..SPL-1), 16 bytes of two each; G8: subvectors 2 q, 2 q + 1 of each group
@@ -1127,17 +1120,9 @@ __device__ __forceinline__ void dn_seg_body(const LayerDev& L, const MoeBufs& B,
 #pragma unroll
                 for (int v = 0; v < NB / 2; ++v) sc[i][v] = sn[i][v];
             f4_t acc[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
-            seg_item_g8<SPL, NB>(w, bx, sc, book, [&](int half) {
-                if constexpr (SPL == 16) {
-                    load_codes(ne, nt, w);
-                } else {
-                    const size_t row0 = static_cast<size_t>(ne) * H + nt * TR + rg * 32;
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-                        seg_load_half(P.codes_t, KS, row0 >> 6, static_cast<int>(row0 & 63) + 16 * i + r16, blk, half,
-                                      w[i]);
-                }
-                if (half == 0) load_scales(ne, nt, sn);
+            seg_item_g8<SPL, NB>(w, bx, sc, book, [&](int) {
+                load_codes(ne, nt, w);
+                load_scales(ne, nt, sn);
             }, acc);
             if (new_unit) load_b(k + 1, bx);
             const int rts[4] = {rt.x, rt.y, rt.z, rt.w};
@@ -1195,20 +1180,20 @@ __device__ __forceinline__ void dn_seg_body(const LayerDev& L, const MoeBufs& B,
     }
 }
 
-template <int NSUB, bool G8>
+template <bool G8>
 __global__ __launch_bounds__(kSegThreads) void k_dn_seg(LayerDev L, MoeBufs B, int M) {
     __shared__ DnSegLds S;
     touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
     const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
-    dn_seg_body<NSUB, G8, 14, -1>(L, B, M, L.p[2], kk & 1, (gridDim.x / 16) * 8, (kk >> 1) * 8 + x8, S);
+    dn_seg_body<G8, 14, -1>(L, B, M, L.p[2], kk & 1, (gridDim.x / 16) * 8, (kk >> 1) * 8 + x8, S);
 }
 __global__ __launch_bounds__(kSegThreads) void k_dn_seg_mixed(LayerDev L, MoeBufs B, int M) {
     __shared__ DnSegLds S;
     touch_kernargs<sizeof(LayerDev) + sizeof(MoeBufs) + sizeof(int)>();
     const int x8 = blockIdx.x & 7, kk = blockIdx.x >> 3;
     const int chunk = kk & 1, per_type = (gridDim.x / 32) * 8, idx = (kk >> 2) * 8 + x8;
-    if (kk & 2) dn_seg_body<64, false, 14, 1>(L, B, M, L.pb[2][1], chunk, per_type, idx, S);
-    else dn_seg_body<64, false, 8, 0>(L, B, M, L.pb[2][0], chunk, per_type, idx, S);
+    if (kk & 2) dn_seg_body<false, 14, 1>(L, B, M, L.pb[2][1], chunk, per_type, idx, S);
+    else dn_seg_body<false, 8, 0>(L, B, M, L.pb[2][0], chunk, per_type, idx, S);
 }
 
 // SwiGLU of every route, the two chunk planes of g and u added; the output is chunk-planar
@@ -1302,8 +1287,8 @@ static int pf_slots(const LayerDev& L, int M) {
 }
 
 // The LDS-codebook kernels serve layers with 4-dim codebook chunks and the tiled codes
-// (d8/14-bit, H / 8 = 128 or 256, I / 8 = 64 or 128) when every workgroup's units fit
-// its table; others take the tile kernels.
+// (d8/14-bit, H 2048, I 512) when every workgroup's units fit its table; others take the tile
+// kernels.
 static int64_t seg_units_per_wg(const LayerDev& L, int M, int tiles, int per_type) {
     const int64_t MK = static_cast<int64_t>(M) * L.K;
     const int shared = L.has_shared && !L.shared_affine;  // (an affine shared expert has no slot)
@@ -1320,13 +1305,10 @@ int prefill_planes(const LayerDev& L, int M) {
         if (L.p[p].ngrp != 1 && L.p[p].ngrp * 64 != (p < 2 ? L.H : L.I)) return 1;
     }
     if (L.p[0].ngrp != L.p[1].ngrp) return 1;
-    const int gn = L.H / 8, dn = L.I / 8;
-    if ((gn != 128 && gn != 256) || (dn != 64 && dn != 128)) return 1;
-    const int gu_rows = 32 * (8 / (gn / 128));  // output rows of a gate/up item
-    if (L.I % gu_rows || L.H % 256 || L.E + 1 > kSegMaxSlots) return 1;
+    if (L.H != 2048 || L.I != 512 || L.E + 1 > kSegMaxSlots) return 1;
     const int grid = mfma_grid();
-    if (seg_units_per_wg(L, M, L.I / gu_rows, grid / 32 * 8) > kSegTab ||
-        seg_units_per_wg(L, M, L.H / 256, grid / 16 * 8) > kSegTab)
+    if (seg_units_per_wg(L, M, L.I / kGuTile, grid / 32 * 8) > kSegTab ||
+        seg_units_per_wg(L, M, L.H / kDnTile, grid / 16 * 8) > kSegTab)
         return 1;
     return 2;
 }
@@ -1350,29 +1332,14 @@ bool moe_uses_seg_verify(const LayerDev& L, int M) {
     return M > 4 && M <= kMaxRows && L.E == 512 && prefill_planes(L, M) == 2;
 }
 
-template <int NSUB>
-hipError_t launch_gu_seg_t(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
-    return launch(L.p[0].ngrp > 1 ? k_gu_seg<NSUB, true> : k_gu_seg<NSUB, false>, dim3(mfma_grid()), dim3(kSegThreads), 0,
-                  st, L, B, M);
-}
-template <int NSUB>
-hipError_t launch_dn_seg_t(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
-    return launch(L.p[2].ngrp > 1 ? k_dn_seg<NSUB, true> : k_dn_seg<NSUB, false>, dim3(mfma_grid()), dim3(kSegThreads), 0,
-                  st, L, B, M);
-}
-
 hipError_t launch_gate_up_pf(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
     if (L.mixed) {  // (eight workgroup types of 8 XCDs)
         if (mfma_grid() < 64) return hipErrorInvalidValue;
         return launch(k_gu_seg_mixed, dim3(mfma_grid() / 64 * 64), dim3(kSegThreads), 0, st, L, B, M);
     }
-    if (prefill_planes(L, M) == 2) {
-        switch (L.H / 8) {
-            case 128: return launch_gu_seg_t<128>(L, B, M, st);
-            case 256: return launch_gu_seg_t<256>(L, B, M, st);
-            default: return hipErrorInvalidValue;
-        }
-    }
+    if (prefill_planes(L, M) == 2)
+        return launch(L.p[0].ngrp > 1 ? k_gu_seg<true> : k_gu_seg<false>, dim3(mfma_grid()), dim3(kSegThreads), 0, st, L,
+                      B, M);
     return launch(k_gu_pf, dim3(L.I / kPfRows, pf_slots(L, M), 2), dim3(256), 0, st, L, B, M);
 }
 
@@ -1388,11 +1355,9 @@ hipError_t launch_swiglu_pf(const LayerDev& L, const MoeBufs& B, int M, hipStrea
 
 hipError_t launch_down_pf(const LayerDev& L, const MoeBufs& B, int M, hipStream_t st) {
     if (L.mixed) return launch(k_dn_seg_mixed, dim3(mfma_grid()), dim3(kSegThreads), 0, st, L, B, M);
-    if (prefill_planes(L, M) == 2) {
-        if (L.I / 8 == 64) return launch_dn_seg_t<64>(L, B, M, st);
-        if (L.I / 8 == 128) return launch_dn_seg_t<128>(L, B, M, st);
-        return hipErrorInvalidValue;
-    }
+    if (prefill_planes(L, M) == 2)
+        return launch(L.p[2].ngrp > 1 ? k_dn_seg<true> : k_dn_seg<false>, dim3(mfma_grid()), dim3(kSegThreads), 0, st, L,
+                      B, M);
     return launch(k_dn_pf, dim3(L.H / kPfRows, pf_slots(L, M), 1), dim3(256), 0, st, L, B, M);
 }
 
