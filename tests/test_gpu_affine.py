@@ -93,6 +93,20 @@ def test_affine_shared_row_tiles(layers, q38, orc, key, M):
     tol_check(orc, y, wy)
 
 
+@pytest.mark.parametrize("M", [17, 65])
+def test_affine_shared_widest_tiles(gpu, q38, orc, M):
+    """H 4096: eight waves of four M-tiles and two columns, 64 KiB of dynamic LDS in gate/up."""
+    L = AffineLayer(q38, gpu, orc, 11, 4, 128, 0, Is=640, H=4096, I=512, E=64, k=4)
+    try:
+        x = orc.rmsnorm(orc.embed(0x5EED + M, list(range(M)), 4096))
+        y, ex, wt, lg, plan = run_forward(q38, L, L.qdesc, x)
+        wy, wex, wwt, _ = L.oracle(orc, x)
+        assert np.array_equal(ex, wex) and np.array_equal(wt, wwt)
+        tol_check(orc, y, wy)
+    finally:
+        L.close()
+
+
 def test_affine_shared_prefill_width(layers, q38, orc):
     L = layers[(4, 64, 0)]
     M = 40

@@ -181,6 +181,42 @@ def test_tile_variants(gpu, q38, orc, geo, S, T0):
     check_cache(keys, values, k2, v2, wk, wv, T0, S)
 
 
+@pytest.mark.parametrize("geo,S,T0", [
+    # 16 + 2 heads of 256, rows on both sides of the second P.V tile limit: whole dims, then slices
+    (dict(q_heads=16, kv_heads=2, head_dim=256, rotary_dim=64), 23, 24565),
+    (dict(q_heads=16, kv_heads=2, head_dim=256, rotary_dim=64), 23, 32681),   # whole dims of 512-token tiles
+    (dict(q_heads=16, kv_heads=2, head_dim=128, rotary_dim=64), 23, 30001),
+    # many kv heads: few queries each on four score tiles a workgroup (16, then 32 queries)
+    (dict(q_heads=8, kv_heads=8, head_dim=64, rotary_dim=32), 5, 16501),
+    (dict(q_heads=16, kv_heads=8, head_dim=64, rotary_dim=32), 10, 16501),
+    (dict(q_heads=8, kv_heads=8, head_dim=128, rotary_dim=32), 3, 16400),
+    (dict(q_heads=16, kv_heads=8, head_dim=128, rotary_dim=32), 10, 16400),
+    (dict(q_heads=8, kv_heads=8, head_dim=256, rotary_dim=32), 3, 16383),     # and 128-token tiles of whole dims
+    (dict(q_heads=16, kv_heads=8, head_dim=256, rotary_dim=32), 10, 16380),
+])
+def test_long_context_variants(gpu, q38, orc, geo, S, T0):
+    """The score and P.V instances of long contexts and of many kv heads: every row, bit for bit,
+    the one-row call's (other instances), and the first and last row against the oracle over the
+    keys and values that the rows before them left in the cache."""
+    L = AttnLayer(seed=10, hidden=256, **geo)
+    rng = np.random.default_rng(T0 + S)
+    cap = T0 + S + 3
+    keys, values = L.random_cache(rng, cap, T0)
+    x = to16(rng.normal(0, 1, (S, L.hidden)), 0)
+    dev = DevAttn(q38, gpu, L, cap)
+    try:
+        cache = dev.cache_dev(keys, values)
+        out = dev.verify(x, cache, T0, T0)
+        k2, v2 = dev.cache_host(cache)
+        for r in range(S):
+            assert np.array_equal(dev.verify(x[r:r + 1], cache, T0 + r, T0 + r)[0], out[r]), r
+    finally:
+        dev.close()
+    for r in (0, S - 1):
+        wout, _, _ = orc.attn_verify(L, x[r:r + 1], k2, v2, T0 + r, T0 + r)
+        tol_check(orc, out[r:r + 1], wout)
+
+
 def test_one_hot_query_reads_its_key_exactly(gpu, q38, orc):
     j = 40
     L = identity_layer(q_rows={j: (0, 3)})

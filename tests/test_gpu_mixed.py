@@ -201,3 +201,27 @@ def test_tensors_on_element_addresses(gpu, q38, mixed_stack):
             assert np.array_equal(u, v)
     finally:
         q38.lib.q38_moe_layer_destroy(L.h)
+
+
+@pytest.mark.parametrize("shared,masked,M", [(1, 1, 16), (0, 0, 9), (0, 1, 5), (0, None, 13), (1, None, 8), (1, 0, 3)])
+def test_banks_without_routes(gpu, q38, orc, shared, masked, M):
+    """One bank masked out of the routing (its workgroups have no unit, or the shared expert's
+    alone), layers without a shared expert, and the row counts between the templates; row r's
+    bits whatever the call's rows."""
+    geo = dict(mixed=1, shared=shared)
+    L = q38.MoeLayer(gpu, q38.desc(**geo), seed=SEED, layer=3)
+    bias = np.zeros(512, np.float32)
+    if masked is not None:
+        bias[masked::2] = -np.inf
+    bias_dev = G.to_dev(bias)
+    q38.check(q38.lib.q38_moe_layer_set_router_bias(L.h, bias_dev.data_ptr()))
+    try:
+        x = orc.rmsnorm(orc.embed(SEED + M, list(range(M)), 2048))
+        y, ex, wt, lg, plan = run_forward(q38, L, L.desc, x)
+        wy, wex, wwt, wlg = orc.moe_layer_synth(oracle_lib.make_desc(**geo), SEED, 3, x, bias=bias)
+        assert np.array_equal(ex, wex) and np.array_equal(wt, wwt)
+        assert masked is None or {int(e) % 2 for e in ex.reshape(-1)} == {1 - masked}
+        tol_check(orc, y, wy)
+        assert np.array_equal(run_forward(q38, L, L.desc, x[:2])[0], y[:2])
+    finally:
+        L.close()

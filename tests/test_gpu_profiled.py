@@ -1,8 +1,8 @@
 """q38_verify_chain_profiled: every phase kernel is timed (start at the phase's first kernel,
-stop at its last), on uniform (one fused gate/up + down + combine kernel at up to 4 rows, as
-for the scale-group stacks),
-mixed (two bank kernels per phase) and per-64-input scale group stacks; the profiled pass
-computes the same values as the plain one."""
+stop at its last), on uniform and per-64-input scale group stacks (one fused gate/up + down +
+combine kernel at up to 4 rows; router, plan, gate/up, SwiGLU, down and combine kernels at 5-16)
+and mixed stacks (the latter at every width); the profiled pass computes the same values as the
+plain one."""
 import ctypes as C
 
 import numpy as np
@@ -14,7 +14,8 @@ from moe_cases import SEED
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kind,M", [("uniform", 4), ("uniform", 1), ("mixed", 16), ("group64", 4), ("group64", 8)])
+@pytest.mark.parametrize("kind,M", [("uniform", 4), ("uniform", 1), ("uniform", 9), ("mixed", 16), ("mixed", 2),
+                                    ("group64", 4), ("group64", 8)])
 def test_profiled_chain(gpu, q38, orc, kind, M):
     import torch
     d = {"uniform": q38.desc(), "mixed": q38.desc(mixed=1), "group64": q38.desc(gu_group=64, down_group=64)}[kind]
