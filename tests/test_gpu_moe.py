@@ -42,7 +42,7 @@ def layer_g64(gpu, q38):
 def test_group64_layer(layer_g64, q38, orc, M):
     """One fp16 scale per 64 inputs (the reference checkpoints' layout) on the config-0
     geometry: rows 1-4 take the four-row MFMA kernels, which scale each K slice's four group
-    partial sums; 16 rows take the grouped VALU kernels. Routing bit-exact, outputs within
+    partial sums; 16 rows take the segmented kernels. Routing bit-exact, outputs within
     the MoE tolerance of the oracle."""
     x = orc.normal(orc.key(SEED, 5, 20), 31 * M, M * 2048, 1.0).reshape(M, 2048)
     y, ex, wt, lg, plan = run_forward(q38, layer_g64, layer_g64.desc, x)
@@ -52,9 +52,24 @@ def test_group64_layer(layer_g64, q38, orc, M):
     tol_check(orc, y, wy)
 
 
-def test_group64_narrow_matches_grouped_kernels(layer_g64, q38, orc):
-    """The same four rows through the four-row kernels (a 4-row call) and the grouped VALU
-    kernels (rows 0-3 of a 5-row call) agree within the MoE tolerance."""
+@pytest.mark.parametrize("M", [1, 4, 5, 16, 40])
+def test_group128_layer(gpu, q38, orc, M):
+    """One fp16 scale per 128 inputs: the grouped VALU kernels at every width."""
+    geo = dict(gu_group=128, down_group=128)
+    L = q38.MoeLayer(gpu, q38.desc(**geo), seed=SEED, layer=6)
+    try:
+        x = orc.normal(orc.key(SEED, 6, 20), 29 * M, M * 2048, 1.0).reshape(M, 2048)
+        y, ex, wt, lg, plan = run_forward(q38, L, L.desc, x)
+        wy, wex, wwt, wlg = orc.moe_layer_synth(oracle_lib.make_desc(**geo), SEED, 6, x)
+        assert np.array_equal(lg, wlg) and np.array_equal(ex, wex) and np.array_equal(wt, wwt)
+        tol_check(orc, y, wy)
+    finally:
+        L.close()
+
+
+def test_group64_narrow_matches_segmented_kernels(layer_g64, q38, orc):
+    """The same four rows through the four-row kernels (a 4-row call) and the segmented kernels
+    (rows 0-3 of a 5-row call) agree within the MoE tolerance."""
     x = orc.normal(orc.key(SEED, 5, 21), 3, 5 * 2048, 1.0).reshape(5, 2048)
     y4 = run_forward(q38, layer_g64, layer_g64.desc, x[:4])[0]
     y5 = run_forward(q38, layer_g64, layer_g64.desc, x)[0]

@@ -167,8 +167,9 @@ def test_prefill_rejects(gpu, q38, orc):
 
 
 # ---------------------------------------------------------------- grouped-scale layouts
-# Layouts the segmented MFMA kernels do not take run at prefill widths on the grouped VALU
-# kernels, in passes of up to 16 of a slot's routes (hot experts take many passes).
+# d8/14-bit layers of 512 experts with 64-input groups run on the segmented MFMA kernels; the
+# layouts these do not take run at prefill widths on the grouped VALU kernels, in passes of up to
+# 16 of a slot's routes (hot experts take many passes).
 
 def test_prefill_512_zipf_group64(gpu, q38, orc):
     """The reference checkpoints' layout (d8/14-bit, one FP16 scale per 64 inputs) at 512 rows
@@ -252,11 +253,12 @@ def test_prefill_grouped_small_layers(gpu, q38, orc, geo, M):
         lay.close()
 
 
-def test_prefill_grouped_matches_verify_rows(gpu, q38, orc):
-    """The same rows through the grouped kernels at prefill width (40 rows) and at verify
-    width (the first 16 rows alone): outputs within the MoE tolerance of each other, routing
-    identical."""
-    d = q38.desc(gu_group=64, down_group=64)
+@pytest.mark.parametrize("group", [64, 128])
+def test_prefill_grouped_matches_verify_rows(gpu, q38, orc, group):
+    """The same rows at prefill width (40 rows) and at verify width (the first 16 rows alone),
+    on the segmented kernels (64-input groups) and the grouped ones (128): outputs within the
+    MoE tolerance of each other, routing identical."""
+    d = q38.desc(gu_group=group, down_group=group)
     L = q38.MoeLayer(gpu, d, seed=SEED, layer=5)
     try:
         x = orc.rmsnorm(orc.embed(SEED, tokens(40), 2048))
