@@ -71,9 +71,10 @@ typedef struct q38_moe_desc {
 /* Device tensors of one layer (uniform geometry). The layer adopts the pointers; the
  * caller keeps them alive for the layer's lifetime. The tensors must be final when the
  * layer is created: creation copies the codebooks (re-laid in 4-dim chunks, or derived
- * per-dimension U8 books) and, for layers the <= 4-row kernels serve, the packed codes
- * (tiled); those kernels read the copies while wider calls read the originals, so a
- * later in-place change would make the two disagree. Expert index E is the shared expert.
+ * per-dimension U8 books) and, for layers the <= 4-row kernels serve (512 experts, H 2048 or
+ * 2560, I 512), the packed codes (tiled). The <= 4-row kernels and the segmented kernels (5-16
+ * rows, and wider calls of d8/14-bit layers) read the copies, the other kernels the originals,
+ * so a later in-place change would make calls disagree. Expert index E is the shared expert.
  *   router       [E, H] bf16                      (SparseMoe::router_,  sparse_moe.hpp:201)
  *   shared_gate  [H] bf16 (w_sg)                  (shared_router_,       sparse_moe.hpp:209)
  *   codes[p]     [E+1, OUT_p, words_p] u32, words_p = ceil(IN_p/D/32)*BITS (E rows without a
@@ -91,7 +92,8 @@ typedef struct q38_moe_weights {
 
 /* Device tensors of a mixed-geometry layer (desc->mixed = 1; hidden 2048, inter 512,
  * one scale per output row). Expert e uses bank e % 2 at index e / 2; the shared expert
- * (index E, even) is the last entry of bank 0.
+ * (index E, even) is the last entry of bank 0. Creation copies the codebooks (the d8 books
+ * decoded to fp16); codes and scales are read in place.
  *   bank 0 (even): codes_d4[p] [E/2+1, OUT_p, ceil(IN_p/4/32)*8] u32 (8-bit codes),
  *                  scales_d4[p] [E/2+1, OUT_p] fp16, books_d4[p] [256, 4] fp16
  *   bank 1 (odd):  codes_d8[p] [E/2, OUT_p, ceil(IN_p/8/32)*14] u32 (14-bit codes),
@@ -202,9 +204,9 @@ void q38_set_fused_layers(int enable);
  * verify-width decode, src/vq_metal_kernels.hpp:564-579, which forms w = q * scale (+ bias)
  * per weight): one 8-byte entry per subvector from a book held whole in LDS, the
  * per-dimension scale applied to the inputs and the bias as a per-row sum. 0: none (the
- * decoded fp16 book on the other kernels); 1 (default): the widths at which they are the faster
- * ones (1-4 rows where the one-launch layer kernel is not taken, 5-16 rows where the segmented
- * kernels are not: other than 512 experts); 2: 1-16 rows.
+ * decoded fp16 book on the other kernels); 1 (default): where neither the one-launch layer (1-4
+ * rows) nor the segmented kernels (5-16 rows of 512 experts) run, which are faster on the decoded
+ * book; 2: 1-16 rows.
  * No counterpart in the reference. */
 void q38_set_u8_native(int mode);
 
@@ -251,8 +253,9 @@ int q38_moe_route(q38_moe_layer* layer, const uint16_t* x, int32_t rows, const q
 /* SparseMoe::forward_verify / forward_prefill (src/sparse_moe.cpp:1953-2171, 2199-2624):
  * y = routed + shared for rows 1..2048 of x. Rows 1..16 take the verify kernels; wider
  * calls (SparseMoe::forward_prefill, include/qwen38/sparse_moe.hpp:68, S <= 2048) take the
- * segmented-GEMM kernels, which need d8/14-bit projections with per-row scales and
- * rows * top_k <= 32768. x, y: device [rows, H] bf16 (may not alias). The expert kernels
+ * segmented-GEMM kernels (d8/14-bit projections with one scale per row or, on 512-expert layers
+ * of H 2048 and I 512, per 64 inputs) or the grouped ones, and need a uniform layer of d8/14,
+ * d4/8 or d2/8 codes and rows * top_k <= 32768. x, y: device [rows, H] bf16 (may not alias). The expert kernels
  * take x as an fp16 MFMA operand: |x| must stay below 65504, and elements below 2^-14 lose
  * relative precision (an RMSNorm output, as in the verify chain, is bounded by sqrt(H) and
  * its small elements weigh nothing in the products). */
@@ -297,15 +300,19 @@ int q38_verify_chain(q38_moe_layer* const* layers, int32_t n_layers, uint16_t* h
                      void* stream);
 
 /* Phase timings of a profiled verify pass (MoeVerifyTimings, include/qwen38/sparse_moe.hpp:
- * 30-36), summed over layers, in milliseconds: the execution time of each phase's kernel,
- * from start/stop events the runtime records at the kernel's own begin and end (the
- * interval a kernel trace reports; launch gaps are not included). */
+ * 30-36), summed over layers, in milliseconds: the time from the
+ * begin of each phase's first kernel to the end of its last one, by events the runtime records
+ * at the kernels' own begin and end (the interval a kernel trace reports; launch gaps between
+ * phases are not included). */
 typedef struct q38_moe_timings {
-    double routing_ms;   /* router logits kernel */
-    double gate_up_ms;   /* gate/up projections (+ top-k + plan on the MFMA path); on layers
+    double routing_ms;   /* router logits; also the affine shared expert's two kernels, and top-k
+                            and plan where the gate/up kernel does not form them itself */
+    double gate_up_ms;   /* gate/up projections (with top-k and plan on the kernels of 1-4 rows and
+                            of per-row scales outside the segmented path); on layers
                             that run gate/up, down and combine in one kernel (d8/14-bit, H
                             2048, I 512, top-10, per-row scales, rows <= 4), that kernel */
-    double down_ms;      /* down projection (+ SwiGLU on the narrow path); 0 on those layers */
+    double down_ms;      /* SwiGLU (a launch of its own on the segmented and U8 paths, inside the
+                            down kernel on the others) and down projection; 0 on those layers */
     double merge_ms;     /* ordered route reduction + shared gate + residual; 0 on those layers */
     int32_t layers;
     int32_t reserved;

@@ -18,11 +18,11 @@
 // (8 KiB of 8-bit weights per wave, the scales, half of the inputs) is issued before the first
 // product, so that a whole projection is in flight at once; the products themselves are a few
 // hundred matrix cycles per wave. Beyond 16 rows four M-tiles share the expanded weights, so
-// they are read once per 64 rows instead of once per 16. Measured, 8-bit g64, against dot
-// products on the vector units with the rows staged in LDS: 4 rows by 12,352 x 2048 18.6 ->
-// 13.4 us (2.0 TB/s), by 2048 x 4096 12.5 -> 6.7 us; 23 rows by 9216 x 2048 55 -> 16 us, by
-// 2048 x 4096 59 -> 12 us; the shared expert of 2048 rows, gate and up 604 -> 52 us, down
-// 174 -> 41 us, of 13 rows 24.2 -> 8.8 and 8.9 -> 4.8 us.
+// they are read once per 64 rows instead of once per 16. Measured (kernel traces), 8-bit g64,
+// against dot products on the vector units with the rows staged in LDS: 4 rows by 12,352 x 2048
+// 16.0 -> 10.9 us (2.5 TB/s), by 2048 x 4096 12.0 -> 7.8 us; 23 rows by 9216 x 2048 55 -> 16 us,
+// by 2048 x 4096 58 -> 12 us; the shared expert of 2048 rows, gate and up 601 -> 54 us, down
+// 173 -> 43 us, of 13 rows 23.4 -> 8.2 and 8.5 -> 4.3 us.
 #pragma once
 
 #include "q38_moe_dev.hpp"

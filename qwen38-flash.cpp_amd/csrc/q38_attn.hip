@@ -164,7 +164,7 @@ __device__ __forceinline__ bool attn_unit(int units, int nmc, int* unit, int* mc
 // and tile the max and the float sum of exp(s - max) over the tokens it sees go to B.stats.
 // Latency-bound: every key of the workgroup is in flight before the first product, and the
 // maxima and sums of all M-tiles meet in LDS together (two barriers a workgroup; one 16-query
-// M-tile at a time with three barriers each took 85 us at 23 rows over 30,001 tokens, now 38 us).
+// M-tile at a time with three barriers each took 84 us at 23 rows over 30,001 tokens, now 37 us).
 template <int D, int MT, int NS>
 __global__ __launch_bounds__(256, 2) void k_attn_scores(AttnDev A, AttnBufs B, int S, const uint16_t* __restrict__ keys,
                                                         int64_t cap, int64_t T0, int64_t tpad, int nmc) {
@@ -310,8 +310,8 @@ __global__ __launch_bounds__(256) void k_attn_stats(AttnDev A, AttnBufs B, int S
 // current one computes.
 // Bound by the serial chain of a sub-tile (loads, p, two barriers, products) and, at long
 // contexts, by the bytes of values, scores and partials. With every wave forming every p (an
-// expf and a division each) and 128-token tiles throughout, 23 rows over 30,001 tokens took 128
-// us, now 33 us; 4 rows over 4,096 tokens 15.2 -> 6.0 us.
+// expf and a division each) and 128-token tiles throughout, 23 rows over 30,001 tokens took 127
+// us, now 33 us; 4 rows over 4,096 tokens 15.7 -> 5.7 us.
 template <int D, int DW, int MT, int NS>
 __global__ __launch_bounds__(256) void k_attn_pv(AttnDev A, AttnBufs B, int S, int row0, int rows,
                                                  const uint16_t* __restrict__ values, int64_t cap, int64_t T0,

@@ -86,7 +86,7 @@ __global__ __launch_bounds__(64) void k_gdn_prework(GdnDev G, GdnBufs B, int S, 
 
 // Lane sum of the 32 lanes of each half-wave in float (xor butterfly 16..1), rounded. The
 // recurrence is one chain of such sums per row: with LDS permutes for the exchanges, integer
-// roundings and one row of inputs in flight it took 9.9 us at 4 rows, now 6.4.
+// roundings and one row of inputs in flight it took 9.5 us at 4 rows, now 6.3.
 __device__ __forceinline__ float half_wave_sum(float v) {
     v += xor_lane_f<16>(v);
     v += xor_lane_f<8>(v);

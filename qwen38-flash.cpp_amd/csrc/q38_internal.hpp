@@ -84,7 +84,7 @@ struct ProjDev {
 // Workspace views of one MoE call (rows <= kMaxRows).
 struct MoeBufs {
     uint16_t* x;       // [M, H] bf16 normalised layer input
-    uint16_t* x16;     // [M, H] fp16 copy of x (MFMA operand)
+    uint16_t* x16;     // [M, H] fp16 copy of x (MFMA operand; segmented kernels: [2][M][H / 2])
     float* logits;     // [M, E]
     float* sgate;      // [M] sigmoid(x . w_sg) rounded to bf16
     int32_t* experts;  // [M*K]

@@ -1,9 +1,9 @@
 // q38_moe_grp.hpp — the grouped-scale expert projections (VALU): layers whose scales are per
-// 64-input group in a geometry the MFMA kernels do not take (d4 and d2 projections, wider
-// calls), the reference checkpoints' layout (src/sparse_moe.cpp:641-647). The kernels and
-// their launchers; each codebook dimension is instantiated in a translation unit of its own
-// (q38_moe_grp{8,4,2}.hip), since their many (bits, lanes-per-row, routes) instantiations
-// dominate the build.
+// input group in a layout the MFMA kernels do not take (groups of other than 64 inputs, d4 and d2
+// projections, expert counts or sizes without tiled codes; src/sparse_moe.cpp:641-647). The
+// kernels and their launchers; each codebook dimension is instantiated in a translation unit of
+// its own (q38_moe_grp{8,4,2}.hip), since their many (bits, lanes-per-row, routes)
+// instantiations dominate the build.
 #pragma once
 
 #include "q38_moe_dev.hpp"

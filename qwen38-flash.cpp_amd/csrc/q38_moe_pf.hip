@@ -1,5 +1,7 @@
 // q38_moe_pf.hip — prefill-width sparse MoE (R1-R3, R9): 17..2048 rows per call, the
-// SparseMoe::forward_prefill_impl segmented path (src/sparse_moe.cpp:2199-2624).
+// SparseMoe::forward_prefill_impl segmented path (src/sparse_moe.cpp:2199-2624). Its segmented
+// kernels on LDS codebook chunks (k_gu_seg, k_swiglu_seg, k_dn_seg) also serve 5..16 rows of
+// 512-expert layers and mixed layers at 1..16 rows (moe_uses_seg_verify).
 //
 //   k_logits_rows  router logits, NE router rows per wave held in registers across
 //                  the workgroup's request rows (the per-lane summation contract of the
@@ -694,8 +696,8 @@ __device__ __forceinline__ void seg_mfma(const uint32_t (&w)[2][NW], const uint4
 // the per-row kernels: A = the route rows, B = the weights, so that a lane owns one weight row
 // (column lane & 15), reads that row's scales, and holds its products with routes 4 q .. 4 q + 3.
 // Bound like the per-row kernels by the random LDS gathers, then by the four scaled adds per
-// MFMA. At 2048 rows (512 experts of about 40 routes): gate/up 6,883 -> 330 us and down 2,862
-// -> 205 us against the grouped vector kernels, which still take the other group sizes.
+// MFMA. At 2048 rows (512 experts of about 40 routes): gate/up 6,853 -> 332 us and down 2,849
+// -> 206 us against the grouped vector kernels, which still take the other group sizes.
 // (Two groups of each span at a time: w holds their 7 words, pr the four spans' pairs, pair
 // 2 b + g for group g of span b.)
 __device__ __forceinline__ void seg_pairs(const uint32_t (&w)[7], uint32_t (&pr)[8]) {
@@ -1015,7 +1017,7 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg(LayerDev L, MoeBufs B, i
 }
 // Both banks of a mixed layer in one launch: workgroup types bank x projection x chunk, half of
 // the workgroups each bank (an item costs its gathers, the same number in both). 16 rows: 35 us,
-// and 21 us for the down kernel, against 41 + 26 and 28 + 24 us of 16-row kernels that ran one
+// and 21 us for the down kernel, against 40 + 24 and 26 + 22 us of 16-row kernels that ran one
 // bank after the other, staged their operand rows and, for the d4 bank, cleared the second plane
 // (32 and 19 us from a tiled copy of the codes, which would double the layer's memory).
 __global__ __launch_bounds__(kSegThreads) void k_gu_seg_mixed(LayerDev L, MoeBufs B, int M) {
