@@ -1031,8 +1031,8 @@ __global__ __launch_bounds__(kSegThreads) void k_gu_seg_mixed(LayerDev L, MoeBuf
 }
 
 // Down (I 512: 64 subvectors per row, SPL = 16 per lane quarter, half a code block). One K part:
-// wave rg owns rows 32 rg .. + 31 of a TR = 256-row tile of H. B = the pass's SwiGLU rows (chunk-planar fp16 at sorted positions); outputs at the
-// route index.
+// wave rg owns rows 32 rg .. + 31 of a TR = 256-row tile of H. B = the pass's SwiGLU rows
+// (chunk-planar fp16 at sorted positions); outputs at the route index.
 constexpr int kDnTile = 256;
 struct DnSegLds {  // one static LDS block, as for gate/up
     uint2 book[kSegKent];
